@@ -19,11 +19,13 @@
  *   q8k_kernel     q8k_quantize_ref (quant.c:174-200, q8_32_ref :150-172):
  *                  d = amax / 127, 1 / d, rint, sums of 16 and of 32.
  *
- * A row is one wave: its numbers sit in LDS, the lanes take the elementwise
- * steps and the rotation's pairs, a wave reduction (exact: a maximum) finds
- * the largest magnitude, and lane 0 alone adds the squares in the reference's
- * order - the one step whose rounding depends on order. No multiply-add is
- * fused in this file, as in the reference's build (-ffp-contract=off).
+ * A row of whole words of four is 16 lanes, its numbers in registers
+ * (rows16_kernel); any other row is one wave: its numbers sit in LDS, the
+ * lanes take the elementwise steps and the rotation's pairs, a wave reduction
+ * (exact: a maximum) finds the largest magnitude, and lane 0 alone adds the
+ * squares in the reference's order - the one step whose rounding depends on
+ * order. No multiply-add is fused in this file, as in the reference's build
+ * (-ffp-contract=off), but for squares that are exact in double.
  */
 #pragma clang fp contract(off)
 
@@ -170,6 +172,266 @@ __global__ __launch_bounds__(64 * kRowWaves) void rows_kernel(const RowArgs A)
                  lane);
 }
 
+/* ---- rows of whole 4-number words: 16 lanes a row ---------------------- */
+
+/*
+ * The same rows, four a wave: lane c of a row's 16 holds numbers 64 b + 4 c ..
+ * + 3 for b < NB (head sizes up to 64 NB), so every access is a word of four
+ * numbers and the reductions are DPP steps inside 16 lanes. It takes rows of
+ * whole words (head size and half the rotation multiples of 4, every array
+ * aligned to its word); the kernels above take the rest.
+ *
+ * What bounded the wave-a-row kernel was the serial sum of squares: one lane,
+ * hd double additions behind LDS reads. One token's 32 query rows of 128 took it
+ * 7.2 us and take 4.5 here (two memory round trips and a chain of divisions and
+ * a square root); 512 tokens' rows 14.9 us and 5.4 (16.8 MB in and out: 3.6 us
+ * at the rate of a large copy).
+ */
+constexpr int kRowLanes = 16;
+constexpr int kRowsWg = 256 / kRowLanes;  /* rows a workgroup */
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef int i4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef int16_t s4 __attribute__((ext_vector_type(4)));
+
+template <int CTRL> __device__ __forceinline__ float dpp(float x)
+{
+    return __uint_as_float(
+        __builtin_amdgcn_update_dpp(0u, __float_as_uint(x), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL> __device__ __forceinline__ double dpp(double x)
+{
+    const uint2 u = __builtin_bit_cast(uint2, x);
+    return __builtin_bit_cast(
+        double, make_uint2(__builtin_amdgcn_update_dpp(0u, u.x, CTRL, 0xf, 0xf, false),
+                           __builtin_amdgcn_update_dpp(0u, u.y, CTRL, 0xf, 0xf, false)));
+}
+/* over a row's 16 lanes, in every lane: quad_perm [1, 0, 3, 2], [2, 3, 0, 1],
+   row_ror 8, row_ror 4. In that order each step adds (or compares) the same
+   two numbers in both lanes of a pair, so a sum has the same bits in all 16
+   (row_ror 4 first would pair each quad with another one in each) */
+__device__ __forceinline__ float max16(float x)
+{
+    x = fmaxf(x, dpp<0xB1>(x));
+    x = fmaxf(x, dpp<0x4E>(x));
+    x = fmaxf(x, dpp<0x128>(x));
+    return fmaxf(x, dpp<0x124>(x));
+}
+__device__ __forceinline__ double sum16(double x)
+{
+    x += dpp<0xB1>(x);
+    x += dpp<0x4E>(x);
+    x += dpp<0x128>(x);
+    return x + dpp<0x124>(x);
+}
+
+/*
+ * 1 / sqrtf(mean of squares + eps) of the row in r (zeros past hd), the bits
+ * of the sum in the order of the row (inv_rms above). The sum is taken as a
+ * tree. Every square is exact in double and none is negative, so a sum of hd
+ * of them, in any order, is within hd 2^-53 of the exact one, and the two
+ * orders within hd 2^-52 of each other; with the division's (here a multiply
+ * by 1 / hd's) roundings, mean (1 +- (hd + 2) 2^-51) holds the mean of the
+ * row's order. Where both ends round to the same float - all but one row in
+ * 2^18 at hd 128 - that float is the mean in the row's order too, since
+ * rounding is monotone. Otherwise (and where the row holds a NaN) the row's
+ * lanes take the sum again in its order.
+ */
+template <int NB>
+__device__ __forceinline__ float inv_rms16(const f4 *r, uint32_t hd, float eps, double inv_hd)
+{
+    double ss = 0.0;
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            ss = __builtin_fma((double)r[b][e], (double)r[b][e], ss);
+    const double mean = sum16(ss) * inv_hd;
+    const double off = mean * ((double)(hd + 2) * 0x1p-51);
+    const float lo = (float)(mean - off), hi = (float)(mean + off);
+    float m = lo;
+    if (!(lo == hi)) {
+        /* lanes of other rows of the wave may be off here: each of the 16
+           lanes of this row is on */
+        const uint32_t row0 = threadIdx.x & 48;
+        double so = 0.0;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+            for (uint32_t c = 0; c < kRowLanes && 64 * b + 4 * c < hd; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const double x = (double)__shfl(r[b][e], row0 + c, 64);
+                    so = __builtin_fma(x, x, so);
+                }
+        m = (float)(so / hd);
+    }
+    return 1.0f / sqrtf(m + eps);
+}
+
+/* the rotation of the row's first 2 half numbers by the token's table, or back:
+   through the row's LDS words, since number i's partner i + half may be in
+   another lane */
+template <int NB, bool BACK>
+__device__ __forceinline__ void rotate16(f4 *r, float *lds, uint32_t c, uint32_t hd, uint32_t half,
+                                         const f4 *cs, const f4 *sn)
+{
+    if (half == 0)
+        return;
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        if (64 * b + 4 * c < hd)
+            *(f4 *)(lds + 64 * b + 4 * c) = r[b];
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const uint32_t col = 64 * b + 4 * c;
+        if (col >= 2 * half || col >= hd)
+            continue;
+        const bool up = col >= half;
+        const f4 o = *(const f4 *)(lds + (up ? col - half : col + half));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float x = r[b][e], y = o[e], cc = cs[b][e], ss = sn[b][e];
+            if (!BACK)
+                r[b][e] = up ? y * ss + x * cc : x * cc - y * ss;
+            else
+                r[b][e] = up ? x * cc - y * ss : x * cc + y * ss;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+/* the lane's words of a token's table: column col's angle is col or
+   col - half of it (unused past the rotation) */
+template <int NB>
+__device__ __forceinline__ void load_table(const float *t, uint32_t c, uint32_t half, f4 *x)
+{
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const uint32_t col = 64 * b + 4 * c;
+        x[b] = f4{0, 0, 0, 0};
+        if (col < 2 * half)
+            x[b] = *(const f4 *)(t + (col < half ? col : col - half));
+    }
+}
+
+/* quantize_row for a row in 16 lanes */
+template <int NB>
+__device__ __forceinline__ void put_row16(const f4 *r, uint32_t c, uint32_t hd, int kv, void *dst,
+                                          float *z)
+{
+    if (kv == kI8 || kv == kI16) {
+        float mx = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                mx = fmaxf(mx, fabsf(r[b][e]));
+        mx = max16(mx);
+        const float top = kv == kI16 ? 32767.0f : 127.0f;
+        const float inv = mx > 0.0f ? top / mx : 0.0f;
+        if (c == 0)
+            *z = mx / top;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const uint32_t col = 64 * b + 4 * c;
+            if (col >= hd)
+                continue;
+            if (kv == kI16) {
+                s4 q;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    q[e] = (int16_t)rintf(r[b][e] * inv);
+                *(s4 *)((int16_t *)dst + col) = q;
+            } else {
+                uint32_t q = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    q |= (uint32_t)(uint8_t)(int8_t)rintf(r[b][e] * inv) << (8 * e);
+                *(uint32_t *)((int8_t *)dst + col) = q;
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const uint32_t col = 64 * b + 4 * c;
+        if (col >= hd)
+            continue;
+        if (kv == kF16) {
+            h4 q;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                q[e] = (_Float16)r[b][e];
+            *(h4 *)((_Float16 *)dst + col) = q;
+        } else {
+            *(f4 *)((float *)dst + col) = r[b];
+        }
+    }
+}
+
+/* rows_kernel's rows, 16 lanes each */
+template <int NB>
+__global__ __launch_bounds__(256) void rows16_kernel(const RowArgs A)
+{
+    __shared__ __attribute__((aligned(16))) float sR[kRowsWg][64 * NB];
+    const uint32_t c = threadIdx.x % kRowLanes, w = threadIdx.x / kRowLanes;
+    const uint32_t id = blockIdx.x * kRowsWg + w;
+    if (id >= A.n * A.heads)
+        return;
+    const uint32_t j = id / A.heads, h = id % A.heads, hd = A.hd, half = A.n_rot / 2;
+    const size_t src = (size_t)id * hd;
+    /* everything the row needs, asked for at once */
+    f4 k[NB], v[NB], nw[NB], cs[NB], sn[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const uint32_t col = 64 * b + 4 * c;
+        k[b] = v[b] = nw[b] = f4{0, 0, 0, 0};
+        if (col >= hd)
+            continue;
+        k[b] = *(const f4 *)(A.k + src + col);
+        if (A.v)
+            v[b] = *(const f4 *)(A.v + src + col);
+        if (A.norm)
+            nw[b] = *(const f4 *)(A.norm + col);
+    }
+    load_table<NB>(A.cs + (size_t)j * half, c, half, cs);
+    load_table<NB>(A.sn + (size_t)j * half, c, half, sn);
+    if (A.norm) {
+        const float s = inv_rms16<NB>(k, hd, A.eps, A.inv_hd);
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                k[b][e] = k[b][e] * s * nw[b][e];
+    }
+    rotate16<NB, false>(k, sR[w], c, hd, half, cs, sn);
+    if (!A.kc) {
+        /* the query: in place */
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+            if (64 * b + 4 * c < hd)
+                *(f4 *)(A.k + src + 64 * b + 4 * c) = k[b];
+        return;
+    }
+    if (A.v_norm) {
+        const float s = inv_rms16<NB>(v, hd, A.eps, A.inv_hd);
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                v[b][e] = v[b][e] * s;
+    }
+    const uint32_t p = A.pos0 + j, row = A.ring ? p % A.cap : p;
+    const size_t at = (size_t)h * A.cap + row;
+    const size_t eb = A.kv == kI8 ? 1 : A.kv == kF32 ? 4 : 2;
+    put_row16<NB>(k, c, hd, A.kv, (char *)A.kc + at * hd * eb, A.kz + at);
+    put_row16<NB>(v, c, hd, A.kv, (char *)A.vc + at * hd * eb, A.vz + at);
+}
+
 /*
  * The shift's rows: moved position i of KV head h is read from the copy
  * (rows src_first + i of the copy, mod cap for a ring), written to its new
@@ -257,11 +519,33 @@ hipError_t launch_refresh(const RefreshArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+/* whether p holds whole words of `bytes` */
+static bool aligned(const void *p, size_t bytes) { return (uintptr_t)p % bytes == 0; }
+
+static size_t elem_size(int kv) { return kv == kI8 ? 1 : kv == kF32 ? 4 : 2; }
+
 hipError_t launch_rows(const RowArgs &a, hipStream_t s)
 {
     const uint32_t rows = a.n * a.heads;
     if (rows == 0)
         return hipSuccess;
+    /* rows of whole words of four take 16 lanes each, any number of rows (one
+       token's 7.2 -> 4.5 us, 512 tokens' 14.9 -> 5.4 us) */
+    const size_t word = 4 * elem_size(a.kv);
+    if (a.hd % 4 == 0 && a.n_rot % 8 == 0 && aligned(a.k, 16) && aligned(a.v, 16) &&
+        aligned(a.norm, 16) && aligned(a.cs, 16) && aligned(a.sn, 16) && aligned(a.kc, word) &&
+        aligned(a.vc, word)) {
+        const dim3 grid((rows + kRowsWg - 1) / kRowsWg), block(256);
+        if (a.hd <= 64)
+            hipLaunchKernelGGL(rows16_kernel<1>, grid, block, 0, s, a);
+        else if (a.hd <= 128)
+            hipLaunchKernelGGL(rows16_kernel<2>, grid, block, 0, s, a);
+        else if (a.hd <= 256)
+            hipLaunchKernelGGL(rows16_kernel<4>, grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL(rows16_kernel<8>, grid, block, 0, s, a);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(rows_kernel, dim3((rows + kRowWaves - 1) / kRowWaves),
                        dim3(64 * kRowWaves), 0, s, a);
     return hipGetLastError();

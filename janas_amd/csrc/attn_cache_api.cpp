@@ -109,6 +109,7 @@ extern "C" int janas_attn_cache_write(const struct janas_attn_cache *c,
     a.n = n;
     a.heads = c->n_kv;
     a.hd = c->head_dim;
+    a.inv_hd = 1.0 / a.hd;
     a.n_rot = n_rot;
     a.pos0 = pos0;
     a.cap = c->cap;
@@ -138,6 +139,7 @@ extern "C" int janas_attn_q_prep(float *q, const float *q_norm, float eps,
     a.n = n;
     a.heads = n_head;
     a.hd = head_dim;
+    a.inv_hd = 1.0 / a.hd;
     a.n_rot = n_rot;
     return hip_rc(launch_rows(a, (hipStream_t)stream), "query launch");
 }

@@ -124,6 +124,7 @@ struct RowArgs {
     const float *cs, *sn;  /* n x n_rot / 2 */
     void *kc, *vc;         /* the cache, heads x cap x hd; null: queries */
     float *kz, *vz;        /* heads x cap scales (int8 / int16) */
+    double inv_hd;         /* 1 / hd */
     float eps;
     uint32_t n, heads, hd, n_rot, pos0, cap;
     int kv, ring, v_norm;

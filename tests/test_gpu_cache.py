@@ -135,6 +135,86 @@ def test_q_prep_bitwise(gpu):
     assert qd.cpu().numpy().tobytes() == want.tobytes()
 
 
+def tie_rows(hd):
+    """Rows whose mean of squares, summed in the row's order, lies half way
+    between two floats F and F + ulp (F even, so it rounds to F), while a sum
+    that adds the small squares together first lies above it: x0^2 = hd F,
+    x1^2 = hd ulp(F) / 2, and hd - 2 numbers whose squares are each a quarter
+    of x0^2's last place in double, lost one by one."""
+    rows = []
+    for m in range(2050, 4096, 2):
+        f = np.float32(m * m) / np.float32(hd)     # exact: 24 bits
+        half = float(np.spacing(f)) / 2 * hd       # x1^2
+        tiny = np.spacing(float(m * m)) / 4
+        if np.log2(half) % 2 or np.log2(tiny) % 2 or int(f.view(np.uint32)) & 1:
+            continue
+        rows.append([m, half ** 0.5] + [tiny ** 0.5] * (hd - 2))
+    return np.array(rows, np.float32)
+
+
+@pytest.mark.parametrize("hd,n_rot", [(128, 128), (128, 24), (512, 0)])
+def test_rows_at_rounding_ties(gpu, hd, n_rot):
+    """The norm's sum of squares where another order of it rounds to another
+    float: the bits of the row's order (1 / sqrtf differs in some of the rows)."""
+    r = tie_rows(hd)
+    n = min(len(r), 300)
+    r = r[np.linspace(0, len(r) - 1, n).astype(int)]
+    d = r.astype(np.float64) ** 2
+    order = np.array([np.float32(np.cumsum(x)[-1] / hd) for x in d])
+    other = (d.sum(axis=1, where=np.arange(hd) > 1) + d[:, 0] + d[:, 1]) / hd
+    eps = np.float32(1e-6)
+    inv = [np.float32(1) / np.sqrt(x.astype(np.float32) + eps) for x in (order, other)]
+    assert (inv[0] != inv[1]).any()
+    cs, sn = rope_tables(range(n), n_rot)
+    want = r[:, None].copy()
+    qn = np.ones(hd, np.float32)
+    orc.q_prep(want, cs=cs, sn=sn, n_rot=n_rot, q_norm=qn, eps=1e-6)
+    qd = dev(r[:, None], gpu)
+    jm.attention.q_prep(qd, cs=dev(cs, gpu) if n_rot else None,
+                        sn=dev(sn, gpu) if n_rot else None, n_rot=n_rot,
+                        q_norm=dev(qn, gpu), eps=1e-6)
+    torch.cuda.synchronize()
+    assert qd.cpu().numpy().tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("hd,n_rot,off", [(40, 40, 0), (48, 16, 0), (68, 56, 0), (100, 8, 0),
+                                          (512, 512, 0), (72, 36, 0), (30, 10, 0),
+                                          (128, 128, 1)])
+def test_rows_of_words_and_others(gpu, hd, n_rot, off):
+    """Head sizes that are whole words of four but not of 64, and rows that are
+    not (an odd half, 30 numbers, arrays one number off a word), one row past a
+    workgroup's 16: cache write and query, the same bits."""
+    n, n_kv, cap = 17, 1, 20
+    rng = np.random.default_rng(hd + off)
+    k = rng.standard_normal((n, n_kv, hd)).astype(np.float32)
+    v = rng.standard_normal((n, n_kv, hd)).astype(np.float32)
+    kn = rng.uniform(0.5, 1.5, hd).astype(np.float32)
+    cs, sn = rope_tables(range(n), n_rot)
+
+    def at(x):
+        """x on the device, `off` numbers past an aligned address"""
+        b = torch.empty(x.size + off, dtype=torch.float32, device=gpu)
+        b[off:] = dev(x.reshape(-1), gpu)
+        return b[off:].view(x.shape)
+    kc = np.zeros((n_kv, cap, hd), np.int8)
+    vc, kz, vz = np.zeros_like(kc), np.zeros((n_kv, cap), np.float32), \
+        np.zeros((n_kv, cap), np.float32)
+    orc.cache_write(k.copy(), v.copy(), cs=cs, sn=sn, n_rot=n_rot, pos0=2, kc=kc,
+                    vc=vc, kz=kz, vz=vz, k_norm=kn, v_norm=True, eps=1e-6)
+    c, (gk, gv, gks, gvs) = device_cache(gpu, n_kv, cap, hd, KV_I8)
+    jm.attention.cache_write(c, at(k), at(v), cs=at(cs), sn=at(sn), n_rot=n_rot, pos0=2,
+                             k_norm=at(kn), eps=1e-6, v_norm=True)
+    want = k.copy()
+    orc.q_prep(want, cs=cs, sn=sn, n_rot=n_rot, q_norm=kn, eps=1e-6)
+    qd = at(k)
+    jm.attention.q_prep(qd, cs=at(cs), sn=at(sn), n_rot=n_rot, q_norm=at(kn), eps=1e-6)
+    torch.cuda.synchronize()
+    assert np.array_equal(gk.cpu().numpy(), kc) and np.array_equal(gv.cpu().numpy(), vc)
+    assert gks.cpu().numpy().tobytes() == kz.tobytes()
+    assert gvs.cpu().numpy().tobytes() == vz.tobytes()
+    assert qd.cpu().numpy().tobytes() == want.tobytes()
+
+
 SHIFT_CASES = [
     # n_kv, hd, cap, n_rot, ring, keep, drop, n_pos
     (2, 128, 256, 128, False, 4, 50, 200),
