@@ -338,8 +338,8 @@ int janas_attn_q_prep(float *q, const float *q_norm, float eps,
  * move down by drop, their keys turned back by the angles of drop positions
  * (cs, sn: n_rot / 2 device floats, as the engine computes them:
  * model.c:323-329) and quantized anew; a ring moves the positions it still
- * holds. int8 / int16 caches. Allocates a copy of the moved rows for the
- * call (and synchronizes the stream to free it).
+ * holds. int8 / int16 caches. Synchronizes the stream. A shift by a small
+ * part of the moved rows, or of a ring, allocates a copy of them for the call.
  */
 int janas_attn_cache_shift(const struct janas_attn_cache *c, uint32_t keep,
                            uint32_t drop, uint32_t n_pos, const float *cs,

@@ -432,8 +432,94 @@ __global__ __launch_bounds__(256) void rows16_kernel(const RowArgs A)
     put_row16<NB>(v, c, hd, A.kv, (char *)A.vc + at * hd * eb, A.vz + at);
 }
 
+/* four numbers of a cached row as the word they are kept in */
+template <int KV> struct Word;
+template <> struct Word<kI8> {
+    typedef uint32_t Raw;
+    __device__ static float at(Raw r, int e) { return (float)(int8_t)(r >> (8 * e)); }
+};
+template <> struct Word<kI16> {
+    typedef uint2 Raw;
+    __device__ static float at(Raw r, int e)
+    {
+        return (float)(int16_t)((e < 2 ? r.x : r.y) >> (16 * (e & 1)));
+    }
+};
+
 /*
- * The shift's rows: moved position i of KV head h is read from the copy
+ * shift_kernel's rows, 16 lanes each. A row's lanes take the positions i, i +
+ * stride, i + 2 stride .. of those that move, in that order. In place (the
+ * copy is the cache itself, stride the shift's distance) that is a chain: each
+ * position's row is read, then goes to where the one before it in the chain
+ * came from, and no other chain reads or writes either row - so the moved rows
+ * need no copy. From a copy the stride is all of them: one row each.
+ *
+ * Bound by memory where chains are short: 16352 of 32768 int8 positions of
+ * 8 x 128 moved in 20.4 us (69 MB, 3.4 TB/s), the call 111 -> 31 us; through
+ * four strided copies and a wave a row, a byte a lane, the copies took 20 us,
+ * the rows 58 and the allocation most of the rest.
+ */
+template <int KV, int NB>
+__global__ __launch_bounds__(256) void shift16_kernel(const ShiftArgs A)
+{
+    using W = Word<KV>;
+    typedef typename W::Raw Raw;
+    __shared__ __attribute__((aligned(16))) float sR[kRowsWg][64 * NB];
+    const uint32_t c = threadIdx.x % kRowLanes, w = threadIdx.x / kRowLanes;
+    const uint64_t id = (uint64_t)blockIdx.x * kRowsWg + w;
+    const uint32_t chains = A.stride < A.count ? A.stride : A.count;
+    if (id >= (uint64_t)A.n_kv * chains)
+        return;
+    const uint32_t h = (uint32_t)(id / chains), hd = A.hd, half = A.n_rot / 2;
+    const uint32_t words = hd / 4;
+    f4 cs[NB], sn[NB];
+    load_table<NB>(A.cs, c, half, cs);
+    load_table<NB>(A.sn, c, half, sn);
+    for (uint64_t i = id % chains; i < A.count; i += A.stride) {
+        const uint32_t p = A.first + (uint32_t)i; /* the position as it was */
+        const uint32_t srow = A.ring ? p % A.cap : p - A.copy_first;
+        const uint32_t drow = A.ring ? (p - A.drop) % A.cap : p - A.drop;
+        const size_t sat = (size_t)h * A.copy_rows + srow;
+        const size_t dat = (size_t)h * A.cap + drow;
+        Raw k[NB], v[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            k[b] = v[b] = Raw{};
+            if (16 * b + c < words) {
+                k[b] = ((const Raw *)A.ck)[sat * words + 16 * b + c];
+                v[b] = ((const Raw *)A.cv)[sat * words + 16 * b + c];
+            }
+        }
+        const float z = A.ckz[sat], vz = A.cvz[sat];
+        /* the value row and its scale move as they are, and the key's when
+           there is nothing to turn */
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+            if (16 * b + c < words) {
+                ((Raw *)A.v)[dat * words + 16 * b + c] = v[b];
+                if (half == 0)
+                    ((Raw *)A.k)[dat * words + 16 * b + c] = k[b];
+            }
+        if (c == 0) {
+            A.vz[dat] = vz;
+            if (half == 0)
+                A.kz[dat] = z;
+        }
+        if (half == 0)
+            continue;
+        f4 r[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                r[b][e] = W::at(k[b], e) * z;
+        rotate16<NB, true>(r, sR[w], c, hd, half, cs, sn);
+        put_row16<NB>(r, c, hd, KV, (Raw *)A.k + dat * words, A.kz + dat);
+    }
+}
+
+/*
+ * Rows that are not whole words: moved position i of KV head h is read from the copy
  * (rows src_first + i of the copy, mod cap for a ring), written to its new
  * row, and its key turned back by the shift's angles and quantized anew
  * (model.c:304-377; unrotate_row :263-290).
@@ -551,11 +637,41 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+bool shift_words(const ShiftArgs &a)
+{
+    const size_t word = 4 * elem_size(a.kv);
+    return a.hd % 4 == 0 && a.n_rot % 8 == 0 && aligned(a.k, word) && aligned(a.v, word) &&
+           aligned(a.ck, word) && aligned(a.cv, word) && aligned(a.cs, 16) && aligned(a.sn, 16);
+}
+
+template <int KV> static void shift16(const ShiftArgs &a, hipStream_t s)
+{
+    const uint64_t rows = (uint64_t)a.n_kv * (a.stride < a.count ? a.stride : a.count);
+    const dim3 grid((uint32_t)((rows + kRowsWg - 1) / kRowsWg)), block(256);
+    if (a.hd <= 64)
+        hipLaunchKernelGGL((shift16_kernel<KV, 1>), grid, block, 0, s, a);
+    else if (a.hd <= 128)
+        hipLaunchKernelGGL((shift16_kernel<KV, 2>), grid, block, 0, s, a);
+    else if (a.hd <= 256)
+        hipLaunchKernelGGL((shift16_kernel<KV, 4>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((shift16_kernel<KV, 8>), grid, block, 0, s, a);
+}
+
 hipError_t launch_shift(const ShiftArgs &a, hipStream_t s)
 {
     const uint32_t rows = a.n_kv * a.count;
     if (rows == 0)
         return hipSuccess;
+    if (shift_words(a)) {
+        if (a.kv == kI16)
+            shift16<kI16>(a, s);
+        else
+            shift16<kI8>(a, s);
+        return hipGetLastError();
+    }
+    if (a.stride < a.count)
+        return hipErrorInvalidValue; /* in place: words only */
     hipLaunchKernelGGL(shift_kernel, dim3((rows + kRowWaves - 1) / kRowWaves),
                        dim3(64 * kRowWaves), 0, s, a);
     return hipGetLastError();

@@ -131,7 +131,8 @@ struct RowArgs {
 };
 
 /* Rows a context shift moves (attn_cache.hip). The copy holds copy_rows
-   rows a KV head: rows copy_first .. of the cache, or all of a ring's. */
+   rows a KV head: rows copy_first .. of the cache, or all of a ring's or of
+   the cache itself (in place). */
 struct ShiftArgs {
     void *k, *v;
     float *kz, *vz;
@@ -141,6 +142,8 @@ struct ShiftArgs {
     uint32_t n_kv, hd, cap, n_rot;
     uint32_t first, count; /* positions first .. first + count - 1 move */
     uint32_t drop, copy_first, copy_rows;
+    uint32_t stride;       /* count: each row from the copy; drop: in place,
+                              ck .. cvz the cache's own (words only) */
     int kv, ring;
 };
 
@@ -213,6 +216,9 @@ struct RefreshArgs {
 hipError_t launch_refresh(const RefreshArgs &a, hipStream_t s);
 hipError_t launch_rows(const RowArgs &a, hipStream_t s);
 hipError_t launch_shift(const ShiftArgs &a, hipStream_t s);
+/* whether the shift's rows are whole aligned words of four (shift16_kernel),
+   which a shift in place needs */
+bool shift_words(const ShiftArgs &a);
 hipError_t launch_q8k(const Q8kArgs &a, hipStream_t s);
 
 /* attn_scratch.hip: the device address of the fixed partials array

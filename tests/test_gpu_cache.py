@@ -222,6 +222,17 @@ SHIFT_CASES = [
     (3, 256, 512, 256, True, 0, 100, 700),
     (2, 128, 256, 128, True, 10, 20, 200),
     (1, 96, 32, 0, False, 2, 5, 30),
+    # chains of rows in place: one row each, the last one short, as long as
+    # they get and one longer (through a copy), by one position
+    (2, 40, 300, 40, False, 1, 150, 300),
+    (3, 512, 80, 512, False, 0, 40, 79),
+    (1, 64, 340, 64, False, 0, 20, 340),
+    (1, 64, 341, 64, False, 0, 20, 341),
+    (2, 128, 17, 128, False, 0, 1, 17),
+    (2, 128, 40, 128, False, 0, 1, 40),
+    # rows that are not whole words
+    (2, 30, 60, 10, False, 3, 20, 60),
+    (2, 72, 60, 36, False, 3, 20, 60),
 ]
 
 
