@@ -1,7 +1,8 @@
 /*
  * attn_planes.h - integers of the engine's int8 / int16 caches as exact f16
  * planes, by byte permutes and packed f16 arithmetic: shared by the split
- * and wide kernels (staging a chunk) and the exact prefill's copy pass.
+ * and wide kernels (staging a chunk) and, for int8, the exact prefill's copy
+ * pass.
  * Internal, device code only.
  *
  * A byte b under the exponent byte 0x64 is the half 1024 + b: halves in

@@ -431,6 +431,33 @@ def test_prefill_quantized_cache(gpu, wide, geom):
     assert within(err, quantized_bar(hd), "vs oracle")
 
 
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_prefill_int16_low_planes(gpu, hd):
+    """int16 numbers whose planes f16(x) and x - f16(x) are the largest (8 off,
+    the ends of the range) under queries whose low plane is the largest and of
+    one sign, so that what the products leave out - low plane times low plane,
+    at most 2^-24 of |q x| each - adds up: scores of sum |q x| scale <= 16
+    move by 2^-20, outputs of magnitude up to 1 by 2^-19 and the f32 sums'
+    rounding, inside the FLOAT bar."""
+    h, kvh, n, cap = 4, 2, 130, 300
+    rng = np.random.default_rng(hd)
+    pick = np.array([32767, 32760, 32744, 20488, 16392, -32768, -16392, 8196, 4098], np.int16)
+    k, v = (pick[rng.integers(0, len(pick), (kvh, cap, hd))] for _ in range(2))
+    ks = np.full((kvh, cap), 1.0 / 32768, np.float32)
+    sign = np.where(rng.random((n, h, hd)) < 0.5, -1.0, 1.0)
+    q = (sign * (1.0 + 2.0 ** -11 - 2.0 ** -22)).astype(np.float32)
+    out = torch.full((n, h, hd), float("nan"), device=gpu)
+    with Attention(h, kvh, hd, cap) as a:
+        a.run_dev(janas_amd.KV_I16, [dict(
+            k=to_dev(k, gpu), v=to_dev(v, gpu), ks=to_dev(ks, gpu),
+            vs=to_dev(ks, gpu), q=to_dev(q, gpu), out=out, cap=cap, n=n,
+            pos0=cap - n)], path="prefill")
+        torch.cuda.synchronize()
+    ref = orc.exact(q, k, v, ks, ks, n_head=h, n_kv=kvh, hd=hd, pos0=cap - n,
+                    kv=janas_amd.KV_I16)
+    assert within(abs_err(out.cpu().numpy(), ref), TOL_FLOAT_ABS, "vs exact")
+
+
 @pytest.mark.parametrize("hd", [128, 64, 256])
 @pytest.mark.parametrize("wide", [False, True])
 def test_prefill_quantized_long_prompt_exact(gpu, wide, hd):
