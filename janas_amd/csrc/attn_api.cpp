@@ -56,7 +56,7 @@ struct janas_attn {
     int dev;
     uint32_t cus;         /* compute units of the device */
     hipStream_t stream;
-    /* partials: part_rows rows of (m, l) and of hd values */
+    /* partials: part_rows rows of hd values, then of (m, l), one block */
     float *part_ml, *part_acc;
     uint64_t part_rows;
     /* the stream that last used the partials: a call on another stream
@@ -255,34 +255,42 @@ int part_sync(janas_attn *a, hipStream_t stream)
     return JANAS_ATTN_OK;
 }
 
+void free_part(janas_attn *a)
+{
+    (void)hipFree(a->part_acc);
+    a->part_ml = a->part_acc = nullptr;
+    a->part_rows = 0;
+}
+
 int ensure_part(janas_attn *a, uint64_t rows, hipStream_t stream)
 {
     if (rows <= a->part_rows)
         return JANAS_ATTN_OK;
     /* the stream that used them last, and this one, may still read the
        old ones */
-    if (a->part_ml || a->part_acc) {
+    if (a->part_acc) {
         hipError_t e = hipStreamSynchronize(stream);
         if (e == hipSuccess && a->part_stream && a->part_stream != stream)
             e = hipStreamSynchronize(a->part_stream);
         if (e != hipSuccess)
             return hip_err(e, "synchronize");
-        (void)hipFree(a->part_ml);
-        (void)hipFree(a->part_acc);
-        a->part_ml = a->part_acc = nullptr;
-        a->part_rows = 0;
+        free_part(a);
     }
-    if (hipMalloc(&a->part_ml, rows * 2 * sizeof(float)) != hipSuccess ||
-        hipMalloc(&a->part_acc, rows * a->hd * sizeof(float)) != hipSuccess) {
+    if (hipMalloc(&a->part_acc, rows * (a->hd + 2) * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
-        (void)hipFree(a->part_ml);
-        (void)hipFree(a->part_acc);
-        a->part_ml = a->part_acc = nullptr;
+        a->part_acc = nullptr;
         return JANAS_ATTN_ENOMEM;
     }
+    /* (hd is a multiple of 8: the pairs stay aligned) */
+    a->part_ml = a->part_acc + rows * a->hd;
     a->part_rows = rows;
     return JANAS_ATTN_OK;
 }
+
+/* an instance's partials from its creation on, at least: a prompt of some
+   hundred tokens in a few key segments needs no more, so its first call does
+   not free and allocate (64 us more; creating an instance takes the same time) */
+constexpr uint64_t kPartBytes = 16u << 20;
 
 /* Where a call's partials live: the instance's (grown as needed, ordered
    across streams), or the device's fixed array of the allocation-free
@@ -707,10 +715,7 @@ void calibrate(janas_attn *a)
     a->prof = prof;
     /* the measurement's partials are not kept: back to the size before */
     if (a->part_rows > rows0) {
-        (void)hipFree(a->part_ml);
-        (void)hipFree(a->part_acc);
-        a->part_ml = a->part_acc = nullptr;
-        a->part_rows = 0;
+        free_part(a);
         if (rows0 && ensure_part(a, rows0, a->stream) != JANAS_ATTN_OK)
             (void)hipGetLastError();
     }
@@ -817,6 +822,139 @@ bool prefill_halves(const janas_attn *a, int kv, const SeqDesc &d)
     return wg < a->cus;
 }
 
+/* How a prefill sequence is split: the kernel and the key segments. */
+struct PrefillSplit {
+    bool halves;
+    uint32_t nseg;
+};
+
+/* partial rows of a split sequence */
+uint64_t prefill_rows(const janas_attn *a, const SeqDesc &d, uint32_t nseg)
+{
+    return nseg > 1 ? (uint64_t)d.n * a->n_head * nseg : 0;
+}
+
+/* An estimate of a prefill sequence's microseconds on this device, to choose
+   between splits with: its workgroups take the compute units in rounds,
+   longest rows first, one workgroup a unit (their LDS or registers fill it),
+   a workgroup 4 us and its tiles' time; a split adds a merge of 3 us and the
+   partials written and read back at 5 TB/s. The constants are a fit to 1042
+   prompts of 80 .. 3000 tokens at 0 .. 8000 positions (16 shapes and cache
+   types) with 1 .. 16 segments each, within 10 % of most. */
+double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, bool halves, int exact,
+                        uint32_t nseg)
+{
+    const uint32_t tile = prefill_tile(a->hd, halves, exact);
+    const uint32_t rows = prefill_block_rows(a->hd, halves, exact), R = d.n * a->group;
+    const uint32_t nb = prefill_row_blocks(d.n, a->group, a->hd, halves, exact);
+    const double tile_us = prefill_tile_us(kv, a->hd, halves), fixed_us = 4.0;
+    /* key tiles of row block b, the longest (the latest) first */
+    auto tiles = [&](uint64_t b) -> uint32_t {
+        const uint32_t r0 = (uint32_t)(nb - 1 - b) * rows;
+        const uint32_t r1 = R - r0 < rows ? R - 1 : r0 + rows - 1;
+        const uint32_t first = d.pos0 + r0 / a->group;
+        const uint32_t hi = d.last ? d.end - 1 : d.pos0 + r1 / a->group;
+        const uint32_t lo = a->window && first + 1 > a->window ? first + 1 - a->window : 0;
+        return hi / tile - lo / tile + 1;
+    };
+    const uint64_t per = (uint64_t)a->n_kv * nseg, N = nb * per, cus = a->cus;
+    /* microseconds of the k-th longest workgroup */
+    auto at = [&](uint64_t k) {
+        return ((tiles(k / per) + nseg - 1) / nseg) * tile_us + fixed_us;
+    };
+    const double longest = at(0);
+    const uint64_t rounds = (N + cus - 1) / cus;
+    double us = longest;
+    if (rounds > 1) {
+        const double mean = (tiles(0) + 2.0 * tiles(nb / 2) + tiles(nb - 1)) / 4;
+        /* as if the work were shared evenly, and as if every round took the
+           longest workgroup's time: by how alike the workgroups are */
+        const double even = (nb * a->n_kv * mean * tile_us + N * fixed_us) / cus;
+        const double alike = at(N - 1) / longest;
+        us = std::max(longest, alike * rounds * longest + (1 - alike) * even);
+        /* two rounds: the second's longest follows the shortest of the first
+           that has one to follow */
+        if (rounds == 2)
+            us = (us + std::max(longest, at(2 * cus - N) + at(N - 1))) / 2;
+    }
+    if (nseg > 1)
+        us += 3.0 + prefill_rows(a, d, nseg) * (a->hd + 2) * 8.0 / 5e6;
+    return us;
+}
+
+/* The split of a prefill sequence: prefill_halves' and prefill_segments',
+   unless the estimate of another is shorter by over a tenth. Those two give
+   each compute unit a workgroup at least, and so leave a second round nearly
+   empty where the row blocks do not divide the units (80 of them, 4 segments:
+   320 workgroups for 256 units), and cut no segment below 6 tiles though a
+   short prefix has few; and one round and a half of equal workgroups (a long
+   prompt in a window) is left as it is. Over the estimate's 1042 prompts the
+   choice takes 0.913 of the time (a 300-token int16 chunk at 8000 positions,
+   16 / 2 / 256, 245 -> 154 us; 80 tokens at 1024, 32 / 8 / 128 f16, 28 -> 19),
+   and 1.05 of it at worst; without the tenth it was 0.909, and 1.2 on some.
+   A sequence whose partials (and exact copy) would pass the allocation-free
+   entry point's array keeps the first choice, and so do prompts of three
+   rounds of workgroups, whose last one weighs little. base: the first choice
+   alone. It depends on the sequence and the device alone. */
+PrefillSplit prefill_split(const janas_attn *a, int kv, const SeqDesc &d, int exact, bool base)
+{
+    PrefillSplit sp;
+    sp.halves = !exact && prefill_halves(a, kv, d);
+    sp.nseg = prefill_segments(a, d, sp.halves, exact);
+    if (base || (uint64_t)a->n_kv * prefill_row_blocks(d.n, a->group, a->hd, sp.halves, exact) >=
+                    3ull * a->cus)
+        return sp;
+    const uint64_t copy = 2ull * exact * a->n_kv * (d.end - d.c0 * kChunk) * a->hd * 2 + 512;
+    double best = 0.9 * prefill_estimate(a, kv, d, sp.halves, exact, sp.nseg);
+    for (int hv = !exact && prefill_halves_supported(kv, a->hd); hv >= 0; hv--) {
+        const uint32_t tile = prefill_tile(a->hd, hv == 1, exact);
+        const uint32_t first = a->window && d.pos0 + 1 > a->window ? d.pos0 + 1 - a->window : 0;
+        const uint32_t nt = (d.end - 1) / tile - first / tile + 1;
+        for (uint32_t s = 1; s <= kMaxSegs && s <= nt; s++) {
+            if (s > 1 && copy + 256 + prefill_rows(a, d, s) * (a->hd + 2) * sizeof(float) >
+                             JANAS_ATTN_NOALLOC_BYTES)
+                break;
+            const double us = prefill_estimate(a, kv, d, hv == 1, exact, s);
+            if (us < best) {
+                best = us;
+                sp = PrefillSplit{hv == 1, s};
+            }
+        }
+    }
+    return sp;
+}
+
+/* The splits of a call's sequences: the first choices alone where the partials
+   would otherwise pass the fixed array, or need more rows than the instance
+   has while the stream is captured. */
+int prefill_splits(janas_attn *a, int kv, const janas_attn_seq *seqs, uint32_t n_seqs, int exact,
+                   hipStream_t stream, bool fixed, uint64_t reserve,
+                   std::vector<PrefillSplit> &splits)
+{
+    for (int base = 0; base < 2; base++) {
+        uint64_t rows = 0;
+        for (uint32_t i = 0; i < n_seqs; i++) {
+            SeqDesc d;
+            int rc = describe(a, kv, seqs[i], d);
+            if (rc)
+                return rc;
+            splits[i] = prefill_split(a, kv, d, exact, base);
+            rows += prefill_rows(a, d, splits[i].nseg);
+        }
+        if (fixed) {
+            if (reserve + rows * (a->hd + 2) * sizeof(float) + 256 <= JANAS_ATTN_NOALLOC_BYTES)
+                break;
+        } else {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            if (rows > a->part_rows && hipStreamIsCapturing(stream, &cs) != hipSuccess)
+                (void)hipGetLastError();
+            if (cs == hipStreamCaptureStatusNone)
+                break;
+        }
+    }
+    return JANAS_ATTN_OK;
+}
+
 /* The sequences in launches of up to kMaxSeqs, those that take the
    two-halves kernel first, then the others. exact: the sequences' k and v
    are the exact copies (run_prefill_x) of int8 (1) or int16 (2) caches;
@@ -825,7 +963,11 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
                        const janas_attn_seq *seqs, uint32_t n_seqs, hipStream_t stream,
                        bool fixed, int exact = 0, uint64_t reserve = 0)
 {
-    for (int hv = 1; hv >= 0; hv--) {
+    std::vector<PrefillSplit> splits(n_seqs);
+    int rc = prefill_splits(a, kv, seqs, n_seqs, exact, stream, fixed, reserve, splits);
+    if (rc)
+        return rc;
+    for (int hv = !exact && prefill_halves_supported(kv, a->hd); hv >= 0; hv--) {
         for (uint32_t i = 0; i < n_seqs;) {
             PrefillArgs args;
             memset(&args, 0, sizeof args);
@@ -834,14 +976,14 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
             uint64_t rows = 0;
             for (; i < n_seqs && m < kMaxSeqs; i++) {
                 SeqDesc &d = args.seq[m];
-                int rc = describe(a, kv, seqs[i], d);
+                rc = describe(a, kv, seqs[i], d);
                 if (rc)
                     return rc;
-                if ((!exact && prefill_halves(a, kv, d)) != (hv == 1))
+                if (splits[i].halves != (hv == 1))
                     continue;
                 d.wg0 = args.wg0s[m] = wg;
                 d.mg0 = args.mg0s[m] = mg;
-                d.nseg = prefill_segments(a, d, hv == 1, exact);
+                d.nseg = splits[i].nseg;
                 d.part0 = 0;
                 uint64_t nwg = (uint64_t)a->n_kv * d.nseg *
                                prefill_row_blocks(d.n, a->group, a->hd, hv == 1, exact);
@@ -862,7 +1004,7 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
                 break;
             Parts pt{nullptr, nullptr, fixed};
             if (rows) {
-                int rc = get_parts(a, rows, stream, fixed, pt, reserve);
+                rc = get_parts(a, rows, stream, fixed, pt, reserve);
                 if (rc)
                     return rc;
             }
@@ -893,7 +1035,7 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
             for (uint32_t j = 0; j < m; j++) {
                 if (args.q8k_fused || args.seq[j].nseg > 1)
                     continue;
-                int rc = put_q8k(a, picked[j], 1, stream);
+                rc = put_q8k(a, picked[j], 1, stream);
                 if (rc)
                     return rc;
             }
@@ -1119,10 +1261,11 @@ extern "C" struct janas_attn *janas_attn_create(uint32_t n_head,
         return nullptr;
     }
     /* the partials of a full janas_attn_run block, as the reference
-       allocates them (attention.c:1013) */
+       allocates them (attention.c:1013), and at least kPartBytes */
     uint32_t chunks = (n_ctx + kChunk - 1) / kChunk;
     uint64_t rows = (uint64_t)n_head_kv * (chunks ? chunks : 1) *
                     JANAS_ATTN_MAX_BLOCK * a->group;
+    rows = std::max<uint64_t>(rows, kPartBytes / ((head_dim + 2) * sizeof(float)));
     if (ensure_part(a, rows, a->stream) != JANAS_ATTN_OK) {
         janas_attn_destroy(a);
         return nullptr;
@@ -1139,8 +1282,7 @@ extern "C" void janas_attn_destroy(struct janas_attn *a)
         (void)hipStreamSynchronize(a->stream);
     if (a->part_stream && a->part_stream != a->stream)
         (void)hipStreamSynchronize(a->part_stream);
-    (void)hipFree(a->part_ml);
-    (void)hipFree(a->part_acc);
+    free_part(a);
     (void)hipFree(a->dq_k);
     (void)hipFree(a->dq_v);
     (void)hipFree(a->st_q);

@@ -236,6 +236,9 @@ int prefill_supported(int kv, uint32_t hd);
 uint32_t prefill_row_blocks(uint32_t n, uint32_t group, uint32_t hd, bool halves,
                             int exact = 0);
 uint32_t prefill_tile(uint32_t hd, bool halves, int exact = 0);
+/* query rows of a row block, and a workgroup's microseconds a key tile */
+uint32_t prefill_block_rows(uint32_t hd, bool halves, int exact = 0);
+double prefill_tile_us(int kv, uint32_t hd, bool halves);
 /* 1 when the two-halves kernel takes this element type and head size */
 int prefill_halves_supported(int kv, uint32_t hd);
 /* xcopy_kernel: the exact kernel's copy of an int8 / int16 cache's rows

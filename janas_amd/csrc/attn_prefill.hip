@@ -1868,15 +1868,34 @@ hipError_t launch_prefill_merge(const PrefillArgs &a, uint32_t n_wg, hipStream_t
     return hipGetLastError();
 }
 
+uint32_t prefill_block_rows(uint32_t hd, bool halves, int exact)
+{
+    return halves ? PCfg<128, true>::BLOCK
+         : hd > 256 ? PCfg<512>::BLOCK
+         : hd > 128 ? PCfg<256>::BLOCK
+         : exact == 2 && hd > 64 ? PCfg<128, false, 2>::BLOCK
+         : exact == 2 ? PCfg<64, false, 2>::BLOCK : PCfg<128>::BLOCK;
+}
+
 uint32_t prefill_row_blocks(uint32_t n, uint32_t group, uint32_t hd, bool halves, int exact)
 {
     /* a workgroup takes PCfg::BLOCK of a KV head's n x group rows */
-    const uint64_t block = halves ? PCfg<128, true>::BLOCK
-                         : hd > 256 ? PCfg<512>::BLOCK
-                         : hd > 128 ? PCfg<256>::BLOCK
-                         : exact == 2 && hd > 64 ? PCfg<128, false, 2>::BLOCK
-                         : exact == 2 ? PCfg<64, false, 2>::BLOCK : PCfg<128>::BLOCK;
+    const uint64_t block = prefill_block_rows(hd, halves, exact);
     return (uint32_t)(((uint64_t)n * group + block - 1) / block);
+}
+
+double prefill_tile_us(int kv, uint32_t hd, bool halves)
+{
+    /* measured where the GPU is not full (the clock is then its highest); the
+       halves' two groups take two tiles at a time */
+    const bool f16 = kv == kF16;
+    if (hd > 256)
+        return f16 ? 2.2 : 2.9;
+    if (hd > 128)
+        return f16 ? 2.2 : kv == kI8 ? 3.4 : 2.8;
+    if (hd > 64)
+        return halves ? 0.92 : f16 ? 2.8 : kv == kI8 ? 3.0 : 2.75;
+    return f16 ? 1.85 : kv == kI8 ? 2.0 : 2.5;
 }
 
 hipError_t launch_prefill(int kv, const PrefillArgs &a, hipStream_t s)

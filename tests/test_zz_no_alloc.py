@@ -8,8 +8,10 @@ import pytest
 import torch
 
 import janas_amd
+from attn_helpers import TOL_F16_ABS, TOL_FLOAT_ABS, abs_err, threads, within
 from cases import normal
 from janas_amd import Attention
+from oracle import orc
 
 pytestmark = pytest.mark.gpu
 
@@ -96,6 +98,110 @@ def test_noalloc_refuses_more_than_the_array(gpu, L, fits):
         a.run_dev(janas_amd.KV_F16, [dict(seq, out=want)])
         torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+# (heads, KV heads, hd, n, pos0, window, ring, with last[]): prompts whose
+# segments (or kernel) follow the estimate: two rounds of workgroups a window
+# holds alike, a second round that was nearly empty, a prefix too short for 6
+# tiles a segment, one round and a bit of a causal prompt, the two-halves kernel
+RESPLIT = [(12, 4, 64, 1000, 0, 1024, False, False), (16, 2, 256, 300, 1000, 0, False, True),
+           (32, 8, 128, 80, 1000, 0, False, False), (32, 8, 128, 1432, 0, 0, False, False),
+           (12, 4, 64, 117, 2082, 300, True, False), (6, 3, 200, 251, 700, 0, False, True)]
+
+
+@pytest.mark.parametrize("kv", [janas_amd.KV_F16, janas_amd.KV_I8, janas_amd.KV_I16])
+@pytest.mark.parametrize("case", range(len(RESPLIT)))
+def test_prompt_splits(gpu, kv, case):
+    """A prompt alone, through the entry point without allocation, beside
+    another one, and recorded into a graph by an instance whose partials are too
+    few (it then splits less): the first three the same bits, all of them the
+    restatement's outputs, gated, with its Q8_K blocks those of its output."""
+    h, kvh, hd, n, pos0, window, ring, spans = RESPLIT[case]
+    cap = 1024 if ring else pos0 + n + 3
+    f32 = [normal(1000 + case + i, kvh * cap * hd).reshape(kvh, cap, hd) for i in (0, 7)]
+    scales = [None, None]
+    if kv == janas_amd.KV_F16:
+        cache = [x.astype(np.float16) for x in f32]
+    else:
+        top = 127 if kv == janas_amd.KV_I8 else 32767
+        scales = [(np.abs(x).max(axis=2) / top).astype(np.float32) for x in f32]
+        cache = [np.rint(x / z[..., None]).astype(np.int8 if top == 127 else np.int16)
+                 for x, z in zip(f32, scales)]
+    q = normal(1020 + case, n * h * hd).reshape(n, h, hd)
+    g = normal(1030 + case, n * h * hd).reshape(n, h, hd)
+    last = None
+    if spans:
+        last = np.minimum(pos0 + np.arange(n) // 3 * 3 + 2, pos0 + n - 1).astype(np.uint32)
+    d = dict(k=dev(cache[0], gpu), v=dev(cache[1], gpu), q=dev(q, gpu), gate=dev(g, gpu),
+             cap=cap, n=n, pos0=pos0)
+    if scales[0] is not None:
+        d.update(ks=dev(scales[0], gpu), vs=dev(scales[1], gpu))
+    if spans:
+        d.update(last=dev(last.view(np.int32), gpu), last_max=int(last.max()))
+    nb = h * hd // 256 if h * hd % 256 == 0 else 0
+
+    def seq():
+        s = dict(d, out=torch.full(d["q"].shape, float("nan"), device=gpu))
+        if nb:
+            s["out_q8k"] = torch.zeros((n, nb, 628), dtype=torch.uint8, device=gpu)
+        return s
+    alone, fixed, beside, other, graphed = (seq() for _ in range(5))
+    st = torch.cuda.Stream()
+
+    def instance(n_ctx):
+        a = Attention(h, kvh, hd, n_ctx, 1, janas_amd.FLOAT)
+        a.set_window(window)
+        a.set_ring(ring)
+        return a
+    with instance(cap) as a, instance(256) as small:
+        gate = janas_amd.GATE_ELEM
+        a.run_dev(kv, [alone], gate)
+        a.run_dev(kv, [fixed], gate, path="noalloc")
+        a.run_dev(kv, [dict(other, n=70, last=None), beside], gate)
+        # (the plain split has no segments here; an integer cache's copy allocates)
+        captured = case == 0 and kv == janas_amd.KV_F16
+        if captured:
+            call = small.prepare(kv, [graphed], gate, stream=st.cuda_stream)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=st):
+                call()
+            for _ in range(3):
+                graphed["out"].zero_()
+                torch.cuda.synchronize()
+                with torch.cuda.stream(st):
+                    graph.replay()
+                torch.cuda.synchronize()
+                assert float((graphed["out"] - alone["out"]).abs().max()) <= TOL_F16_ABS
+        torch.cuda.synchronize()
+    assert torch.equal(alone["out"], fixed["out"])
+    assert torch.equal(alone["out"], beside["out"])
+    ref = orc.run(q.astype(np.float32), cache[0], cache[1], scales[0], scales[1], n_head=h,
+                  n_kv=kvh, hd=hd, pos0=pos0, kv=kv, window=window, ring=ring, last=last,
+                  threads=threads(), block=64)
+    orc.gate(ref, g)
+    bar = TOL_F16_ABS if kv == janas_amd.KV_F16 else TOL_FLOAT_ABS
+    assert within(abs_err(alone["out"].cpu().numpy(), ref), bar, "vs oracle")
+    if nb:
+        want = orc.q8k_quantize(alone["out"].cpu().numpy().reshape(n, h * hd))
+        assert alone["out_q8k"].cpu().numpy().tobytes() == want.tobytes()
+
+
+def test_noalloc_prompts_that_pass_the_array_together(gpu):
+    """Prompts whose segments' partials fit the array one by one and not
+    together split less there, and still run: outputs within the f16 bar of
+    janas_attn_run_dev's."""
+    h, kvh, hd, n, L = 12, 4, 64, 1000, 1000
+    k = dev(normal(171, kvh * L * hd).reshape(kvh, L, hd).astype(np.float16), gpu)
+    q = dev(normal(173, n * h * hd).reshape(n, h, hd), gpu)
+    outs = [[torch.full_like(q, float("nan")) for _ in range(12)] for _ in range(2)]
+    with Attention(h, kvh, hd, L) as a:
+        for path, out in zip(("auto", "noalloc"), outs):
+            a.run_dev(janas_amd.KV_F16, [dict(k=k, v=k, q=q, out=o, cap=L, n=n, pos0=0)
+                                         for o in out], path=path)
+        torch.cuda.synchronize()
+    for x, y in zip(*outs):
+        assert float((x - y).abs().max()) <= TOL_F16_ABS
 
 
 def test_noalloc_under_graph_capture(gpu):
