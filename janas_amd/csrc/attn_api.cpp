@@ -452,6 +452,9 @@ int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
             tiles = std::max<uint64_t>(tiles, ((uint64_t)seqs[s0 + i].n * a->group + tr - 1) / tr);
         args.mt = split_mt(kv, a->hd, (uint32_t)std::min<uint64_t>(tiles, kSplitMaxMt));
         args.once = 1;
+        /* one chunk a sequence: no merge, unless it has Q8_K blocks to make or
+           chunks to count */
+        bool direct = kernels == 3 && split_direct(a->hd) && !q8k && g_skip <= 0;
         uint32_t wg = 0, mg = 0;
         /* merge workgroups a (token, head), or a token's blocks */
         const uint32_t nd = (a->hd + args.merge_cols - 1) / args.merge_cols;
@@ -468,6 +471,7 @@ int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
             args.once &= d.rtiles == 1;
             uint64_t nwg = (uint64_t)a->n_kv * d.span * d.rtiles;
             uint64_t nmg = q8k ? (uint64_t)d.n * nb : (uint64_t)d.n * a->n_head * nd;
+            direct &= d.span == 1;
             if (wg + nwg > 0x7FFFFFFFu || mg + nmg > 0x7FFFFFFFu)
                 return JANAS_ATTN_ERANGE;
             wg += (uint32_t)nwg;
@@ -480,6 +484,8 @@ int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
             return rc;
         args.n_seqs = m;
         args.n_wg = wg;
+        if (direct)
+            args.merge_cols = kMergeNone;
         fill_args(a, kv, args, gate_mode, pt);
         if (kernels & 1) {
             ProfEv *ev = fixed ? nullptr : prof_begin(a, 0, stream);
@@ -488,7 +494,7 @@ int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
             if (e != hipSuccess)
                 return hip_err(e, "split launch");
         }
-        if (kernels & 2) {
+        if ((kernels & 2) && !direct) {
             ProfEv *ev = fixed ? nullptr : prof_begin(a, 1, stream);
             hipError_t e = launch_merge(args, mg, stream);
             prof_end(ev, stream);

@@ -23,6 +23,8 @@ constexpr uint32_t kWideRows = 16;
 inline uint32_t split_tile_rows(uint32_t hd) { return hd > 256 ? kWideRows : kTileRows; }
 /* merge_cols of a merge that also puts its outputs into Q8_K blocks */
 constexpr uint32_t kMergeQ8k = 256;
+/* and of a launch without a merge */
+constexpr uint32_t kMergeNone = 0;
 /* sequences one launch takes (by value in its arguments) */
 constexpr uint32_t kMaxSeqs = 16;
 /* merge workgroups a launch keeps at least when it takes 128 columns a
@@ -65,7 +67,9 @@ struct SplitArgs {
     uint32_t mt;           /* split kernel: row tiles a workgroup (1 or 2;
                               split_mt) */
     uint32_t merge_cols;   /* 32 or 128 columns a merge workgroup, or
-                              kMergeQ8k: one Q8_K block of 256 outputs */
+                              kMergeQ8k: one Q8_K block of 256 outputs, or
+                              kMergeNone: every sequence sees one chunk and
+                              the split kernel writes the outputs */
     uint32_t n_head, n_kv, group, hd, window;
     float scale;
     int ring;
@@ -196,6 +200,9 @@ int split_supported(int kv, uint32_t hd);
 /* row tiles a split-kernel workgroup takes for a launch whose largest
    sequence has `tiles` row tiles (SplitArgs::mt). */
 uint32_t split_mt(int kv, uint32_t hd, uint32_t tiles);
+/* whether the split kernel of this head size can write the outputs itself
+   (kMergeNone) */
+inline bool split_direct(uint32_t hd) { return hd <= 256; }
 /* attn_wide.hip: the split kernel for head sizes 264 .. 512 (8- and 16-bit
    caches); launch_split hands those to it. */
 hipError_t launch_wide(int kv, const SplitArgs &a, hipStream_t s);

@@ -10,7 +10,7 @@ import torch
 import janas_amd
 from attn_helpers import (KV_F16, KV_F32, KV_I8, TOL_F16_ABS, TOL_F32_REL,
                           TOL_FLOAT_ABS, abs_err, config, oracle_out, rel_err, within)
-from cases import CASES, KV_I16, call_kwargs, make_inputs
+from cases import CASES, KV_I16, call_kwargs, make_inputs, normal
 from janas_amd import Attention
 from oracle import orc
 
@@ -396,3 +396,66 @@ def test_large_block_ragged_sequences(gpu):
                                         n=1, pos0=p0 + j)], path="split")
             torch.cuda.synchronize()
             assert torch.equal(d["out"].view(torch.int32), one.view(torch.int32))
+
+
+@pytest.mark.parametrize("gate", [janas_amd.GATE_NONE, janas_amd.GATE_ELEM, janas_amd.GATE_HEAD])
+@pytest.mark.parametrize("kv,scores", [(janas_amd.KV_F16, janas_amd.FLOAT),
+                                       (janas_amd.KV_I8, janas_amd.FLOAT),
+                                       (janas_amd.KV_I8, janas_amd.INT16),
+                                       (janas_amd.KV_I16, janas_amd.FLOAT),
+                                       (janas_amd.KV_F32, janas_amd.FLOAT)])
+def test_one_chunk_equals_its_merge(gpu, kv, scores, gate):
+    """A call that sees one chunk writes its output from the split kernel: the
+    bits of the two kernels one at a time (partials, then the merge) - one
+    token and blocks, rows past a tile, chunks past the first (a window, a
+    ring), last[], several sequences of which some see more chunks."""
+    shapes = [(8, 2, 64, 0), (6, 2, 128, 0), (5, 1, 40, 0), (16, 2, 128, 40)]
+    if kv != janas_amd.KV_F32:
+        shapes.append((16, 2, 256, 0))
+    for h, n_kv, hd, window in shapes:
+        if scores == janas_amd.INT16 and hd % 16:
+            continue
+        cap = 768
+        def numbers(seed):
+            x = normal(seed, n_kv * cap * hd).reshape(n_kv, cap, hd)
+            if kv == janas_amd.KV_F16:
+                return torch.from_numpy(x.astype(np.float16)).to(gpu), None
+            if kv == janas_amd.KV_F32:
+                return torch.from_numpy(x.astype(np.float32)).to(gpu), None
+            top = 127 if kv == janas_amd.KV_I8 else 32767
+            z = (np.abs(x).max(axis=2) / top).astype(np.float32)
+            q = np.rint(x / z[..., None]).astype(np.int8 if top == 127 else np.int16)
+            return torch.from_numpy(q).to(gpu), torch.from_numpy(z).to(gpu)
+        k, ks = numbers(hd + h)
+        v, vs = numbers(hd + h + 1)
+        calls = [[(1, 0, None)], [(1, 255, None)], [(64, 192, None)], [(3, 100, [150, 150, 255])],
+                 [(1, 30, None), (5, 254, None), (2, 7, None)], [(1, 600, None), (1, 5, None)]]
+        if window:
+            calls = [[(1, 511, None)], [(2, 600, None)], [(1, 767, None), (9, 290, None)]]
+        for ring in ([False, True] if window else [False]):
+            with Attention(h, n_kv, hd, cap, 1, scores) as a:
+                a.set_window(window)
+                a.set_ring(ring)
+                for ci, call in enumerate(calls):
+                    outs = []
+                    for paths in (("auto",), ("split-kernel", "merge-kernel")):
+                        seqs = []
+                        for i, (n, pos0, last) in enumerate(call):
+                            q = normal(7 + i, n * h * hd).reshape(n, h, hd).astype(np.float32)
+                            g = normal(9 + i, n * h * hd).reshape(n, h, hd).astype(np.float32)
+                            if gate == janas_amd.GATE_HEAD:
+                                g = g[:, :, 0].copy()
+                            q = torch.from_numpy(q).to(gpu)
+                            d = dict(k=k, v=v, ks=ks, vs=vs, q=q, cap=cap, n=n, pos0=pos0,
+                                     out=torch.full_like(q, float("nan")),
+                                     gate=torch.from_numpy(g).to(gpu))
+                            if last:
+                                d.update(last=torch.tensor(last, dtype=torch.int32, device=gpu),
+                                         last_max=last[-1])
+                            seqs.append(d)
+                        for path in paths:
+                            a.run_dev(kv, seqs, gate, path=path)
+                        torch.cuda.synchronize()
+                        outs.append([d["out"].cpu().numpy().view(np.int32) for d in seqs])
+                    for x, y in zip(*outs):
+                        assert np.array_equal(x, y), (h, n_kv, hd, window, ring, ci)
