@@ -323,6 +323,7 @@ __global__ __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(D <= 1
     issue(1);
     __builtin_amdgcn_sched_barrier(0);
 
+    const float neg1 = minus_one();
     /* ---- the query planes: scaled by 2^e so that the row's largest |q|
        lies in [2^13, 2^14), split into f16 hi + lo, into LDS ---- */
 #pragma unroll
@@ -372,11 +373,12 @@ __global__ __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(D <= 1
         const float up = ldexpf(1.0f, ex);
         if (qrow[h] < kTileRows) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                _Float16 hi, lo;
-                split_hl(ok && qcol[h] < hd ? x[e] * up : 0.0f, hi, lo);
-                sQ[2 * tr][qcol[h] + e] = hi;
-                sQ[2 * tr + 1][qcol[h] + e] = lo;
+            for (int e = 0; e < 4; e += 2) {
+                const bool in = ok && qcol[h] < hd;
+                h2 hi, lo;
+                split_hl2(in ? x[e] * up : 0.0f, in ? x[e + 1] * up : 0.0f, neg1, hi, lo);
+                *(h2 *)&sQ[2 * tr][qcol[h] + e] = hi;
+                *(h2 *)&sQ[2 * tr + 1][qcol[h] + e] = lo;
             }
             if (qcol[h] == 0)
                 sQs[tr] = ldexpf(1.0f, -ex);
@@ -426,14 +428,10 @@ __global__ __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(D <= 1
             *(h8 *)(rb + 16 * slot<D>(cb / 8, row)) = Elem<kI8>::widen(x.x, x.y);
             *(h8 *)(rb + 16 * slot<D>(cb / 8 + 1, row)) = Elem<kI8>::widen(x.z, x.w);
         } else {
-            h4 hi, lo;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                _Float16 a, b;
-                split_hl(__uint_as_float(x0[e]), a, b);
-                hi[e] = a;
-                lo[e] = b;
-            }
+            h2 a, b, c, d;
+            split_hl2(__uint_as_float(x0[0]), __uint_as_float(x0[1]), neg1, a, c);
+            split_hl2(__uint_as_float(x0[2]), __uint_as_float(x0[3]), neg1, b, d);
+            const h4 hi = {a[0], a[1], b[0], b[1]}, lo = {c[0], c[1], d[0], d[1]};
             const uint32_t u = cb / 32, half = (cb / 16) & 1;
             *(h4 *)(rb + 16 * slot<D>(u, row) + 8 * half) = hi;
             *(h4 *)(rb + S::PLB + 16 * slot<D>(u, row) + 8 * half) = lo;
