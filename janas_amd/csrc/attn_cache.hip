@@ -251,7 +251,7 @@ __device__ __forceinline__ float inv_rms16(const f4 *r, uint32_t hd, float eps, 
     const double off = mean * ((double)(hd + 2) * 0x1p-51);
     const float lo = (float)(mean - off), hi = (float)(mean + off);
     float m = lo;
-    if (!(lo == hi)) {
+    if (__builtin_expect(!(lo == hi), 0)) {
         /* lanes of other rows of the wave may be off here: each of the 16
            lanes of this row is on */
         const uint32_t row0 = threadIdx.x & 48;
@@ -319,11 +319,11 @@ __device__ __forceinline__ void load_table(const float *t, uint32_t c, uint32_t 
 }
 
 /* quantize_row for a row in 16 lanes */
-template <int NB>
-__device__ __forceinline__ void put_row16(const f4 *r, uint32_t c, uint32_t hd, int kv, void *dst,
+template <int NB, int kv>
+__device__ __forceinline__ void put_row16(const f4 *r, uint32_t c, uint32_t hd, void *dst,
                                           float *z)
 {
-    if (kv == kI8 || kv == kI16) {
+    if constexpr (kv == kI8 || kv == kI16) {
         float mx = 0.0f;
 #pragma unroll
         for (int b = 0; b < NB; b++)
@@ -373,8 +373,10 @@ __device__ __forceinline__ void put_row16(const f4 *r, uint32_t c, uint32_t hd, 
     }
 }
 
-/* rows_kernel's rows, 16 lanes each */
-template <int NB>
+/* rows_kernel's rows, 16 lanes each; KV the cache's type, or -1: queries (a
+   type's test in the kernel was a jump over the others' code, a miss of the
+   instruction cache: four layers' decode step 106.7 -> 105.4 us) */
+template <int NB, int KV>
 __global__ __launch_bounds__(256) void rows16_kernel(const RowArgs A)
 {
     __shared__ __attribute__((aligned(16))) float sR[kRowsWg][64 * NB];
@@ -409,7 +411,7 @@ __global__ __launch_bounds__(256) void rows16_kernel(const RowArgs A)
                 k[b][e] = k[b][e] * s * nw[b][e];
     }
     rotate16<NB, false>(k, sR[w], c, hd, half, cs, sn);
-    if (!A.kc) {
+    if constexpr (KV < 0) {
         /* the query: in place */
 #pragma unroll
         for (int b = 0; b < NB; b++)
@@ -427,9 +429,9 @@ __global__ __launch_bounds__(256) void rows16_kernel(const RowArgs A)
     }
     const uint32_t p = A.pos0 + j, row = A.ring ? p % A.cap : p;
     const size_t at = (size_t)h * A.cap + row;
-    const size_t eb = A.kv == kI8 ? 1 : A.kv == kF32 ? 4 : 2;
-    put_row16<NB>(k, c, hd, A.kv, (char *)A.kc + at * hd * eb, A.kz + at);
-    put_row16<NB>(v, c, hd, A.kv, (char *)A.vc + at * hd * eb, A.vz + at);
+    constexpr size_t eb = KV == kI8 ? 1 : KV == kF32 ? 4 : 2;
+    put_row16<NB, KV>(k, c, hd, (char *)A.kc + at * hd * eb, A.kz + at);
+    put_row16<NB, KV>(v, c, hd, (char *)A.vc + at * hd * eb, A.vz + at);
 }
 
 /* four numbers of a cached row as the word they are kept in */
@@ -514,7 +516,7 @@ __global__ __launch_bounds__(256) void shift16_kernel(const ShiftArgs A)
             for (int e = 0; e < 4; e++)
                 r[b][e] = W::at(k[b], e) * z;
         rotate16<NB, true>(r, sR[w], c, hd, half, cs, sn);
-        put_row16<NB>(r, c, hd, KV, (Raw *)A.k + dat * words, A.kz + dat);
+        put_row16<NB, KV>(r, c, hd, (Raw *)A.k + dat * words, A.kz + dat);
     }
 }
 
@@ -610,6 +612,20 @@ static bool aligned(const void *p, size_t bytes) { return (uintptr_t)p % bytes =
 
 static size_t elem_size(int kv) { return kv == kI8 ? 1 : kv == kF32 ? 4 : 2; }
 
+template <int KV> static hipError_t rows16(const RowArgs &a, hipStream_t s)
+{
+    const dim3 grid((a.n * a.heads + kRowsWg - 1) / kRowsWg), block(256);
+    if (a.hd <= 64)
+        hipLaunchKernelGGL((rows16_kernel<1, KV>), grid, block, 0, s, a);
+    else if (a.hd <= 128)
+        hipLaunchKernelGGL((rows16_kernel<2, KV>), grid, block, 0, s, a);
+    else if (a.hd <= 256)
+        hipLaunchKernelGGL((rows16_kernel<4, KV>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((rows16_kernel<8, KV>), grid, block, 0, s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_rows(const RowArgs &a, hipStream_t s)
 {
     const uint32_t rows = a.n * a.heads;
@@ -621,16 +637,19 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s)
     if (a.hd % 4 == 0 && a.n_rot % 8 == 0 && aligned(a.k, 16) && aligned(a.v, 16) &&
         aligned(a.norm, 16) && aligned(a.cs, 16) && aligned(a.sn, 16) && aligned(a.kc, word) &&
         aligned(a.vc, word)) {
-        const dim3 grid((rows + kRowsWg - 1) / kRowsWg), block(256);
-        if (a.hd <= 64)
-            hipLaunchKernelGGL(rows16_kernel<1>, grid, block, 0, s, a);
-        else if (a.hd <= 128)
-            hipLaunchKernelGGL(rows16_kernel<2>, grid, block, 0, s, a);
-        else if (a.hd <= 256)
-            hipLaunchKernelGGL(rows16_kernel<4>, grid, block, 0, s, a);
-        else
-            hipLaunchKernelGGL(rows16_kernel<8>, grid, block, 0, s, a);
-        return hipGetLastError();
+        switch (a.kc ? a.kv : -1) {
+        case -1:
+            return rows16<-1>(a, s);
+        case kI8:
+            return rows16<kI8>(a, s);
+        case kI16:
+            return rows16<kI16>(a, s);
+        case kF16:
+            return rows16<kF16>(a, s);
+        case kF32:
+            return rows16<kF32>(a, s);
+        }
+        return hipErrorInvalidValue;
     }
     hipLaunchKernelGGL(rows_kernel, dim3((rows + kRowWaves - 1) / kRowWaves),
                        dim3(64 * kRowWaves), 0, s, a);
