@@ -14,7 +14,9 @@
 #include <sys/stat.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -970,7 +972,7 @@ PrefillSplit prefill_split(const janas_attn *a, int kv, const SeqDesc &d, int ex
    has while the stream is captured. */
 int prefill_splits(janas_attn *a, int kv, const janas_attn_seq *seqs, uint32_t n_seqs, int exact,
                    hipStream_t stream, bool fixed, uint64_t reserve,
-                   std::vector<PrefillSplit> &splits)
+                   PrefillSplit *splits)
 {
     for (int base = 0; base < 2; base++) {
         uint64_t rows = 0;
@@ -1004,8 +1006,11 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
                        const janas_attn_seq *seqs, uint32_t n_seqs, hipStream_t stream,
                        bool fixed, int exact = 0, uint64_t reserve = 0)
 {
-    std::vector<PrefillSplit> splits(n_seqs);
-    int rc = prefill_splits(a, kv, seqs, n_seqs, exact, stream, fixed, reserve, splits);
+    /* (no exception may leave the C entry point) */
+    std::unique_ptr<PrefillSplit[]> splits(new (std::nothrow) PrefillSplit[n_seqs]);
+    if (!splits)
+        return JANAS_ATTN_ENOMEM;
+    int rc = prefill_splits(a, kv, seqs, n_seqs, exact, stream, fixed, reserve, splits.get());
     if (rc)
         return rc;
     for (int hv = !exact && prefill_halves_supported(kv, a->hd); hv >= 0; hv--) {

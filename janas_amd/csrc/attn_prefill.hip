@@ -1028,10 +1028,10 @@ __global__ __launch_bounds__(PCfg<D>::W * 64) void prefill_dma_kernel(const Pref
  * the nearest f16, and what is left, at most 8), and the query and the
  * weights as two f16 planes each (x = hi + lo, 22 significant bits), so each
  * product is exact in the matrix core and summed in f32. Over int16 three of
- * the four plane products are made: both low planes are at most 2^-12 of
- * their numbers, so low times low is at most 2^-24 of the product, half a unit
- * of the f32 sum it would enter (with x >> 8 and x & 255 as planes it was
- * 2^-20, and made). A 3001-token prompt at 16 / 2 / 256 in a window of 1024 265
+ * the four plane products are made: both low planes are at most 2^-11 of
+ * their numbers, so low times low is at most 2^-22 of the product, as much as
+ * the query's and the weights' two planes leave of them (x & 255 as the low
+ * plane is no such part of a small x: low times low was made). A 3001-token prompt at 16 / 2 / 256 in a window of 1024 265
  * -> 231 us, 4096 tokens at 32 / 8 / 128 523 -> 444 us, the error against 64
  * bits 9.4e-7 -> 8.7e-7 and 8.6e-7 -> 8.0e-7. The scales stay f32:
  *   score   s = (sum_i q'_i k_i) * ks[p] * 2^-e,  q' = q * scale * log2(e) * 2^e
