@@ -280,9 +280,8 @@ int ensure_part(janas_attn *a, uint64_t rows, hipStream_t stream)
             return hip_err(e, "synchronize");
         free_part(a);
     }
-    /* whole pages of 2 MiB, none of the tail in small ones: creating an
-       instance takes 35 - 140 us less (as much as two arrays did), a ragged
-       decode of 8 sequences 31.7 us for 31.9 - 32.2 */
+    /* whole pages of 2 MiB, none of the tail in small ones: a ragged decode of
+       8 sequences 31.7 - 31.8 us for 31.9 - 32.2 */
     const uint64_t bytes = (rows * (a->hd + 2) * sizeof(float) + kPage - 1) / kPage * kPage;
     if (hipMalloc(&a->part_acc, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -297,7 +296,8 @@ int ensure_part(janas_attn *a, uint64_t rows, hipStream_t stream)
 
 /* an instance's partials from its creation on, at least: a prompt of some
    hundred tokens in a few key segments needs no more, so its first call does
-   not free and allocate (64 us more; creating an instance takes the same time) */
+   not free and allocate (64 us; creating an instance that needs less takes 30
+   - 50 us more) */
 constexpr uint64_t kPartBytes = 16u << 20;
 
 /* Where a call's partials live: the instance's (grown as needed, ordered
