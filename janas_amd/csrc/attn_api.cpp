@@ -836,26 +836,16 @@ bool prefill_halves(const janas_attn *a, int kv, const SeqDesc &d)
     return wg < a->cus;
 }
 
-/* How a prefill sequence is split: the kernel, the key segments of a split
-   row block, and how many of a KV head's row blocks are split: all of them, or
-   the last ones to be dispatched (the first rows). */
+/* How a prefill sequence is split: the kernel and the key segments. */
 struct PrefillSplit {
     bool halves;
-    uint32_t nseg, blocks;
+    uint32_t nseg;
 };
 
-/* the tokens whose row blocks are split (they are whole tokens: the split
-   covers all rows, or blocks of whole tokens), and their partial rows */
-uint32_t prefill_tokens(const janas_attn *a, const SeqDesc &d, const PrefillSplit &sp, int exact)
+/* partial rows of a split sequence */
+uint64_t prefill_rows(const janas_attn *a, const SeqDesc &d, uint32_t nseg)
 {
-    if (sp.nseg < 2)
-        return 0;
-    const uint64_t rows = (uint64_t)sp.blocks * prefill_block_rows(a->hd, sp.halves, exact);
-    return (uint32_t)std::min<uint64_t>(d.n, rows / a->group);
-}
-uint64_t prefill_rows(const janas_attn *a, const SeqDesc &d, const PrefillSplit &sp, int exact)
-{
-    return (uint64_t)prefill_tokens(a, d, sp, exact) * a->n_head * sp.nseg;
+    return nseg > 1 ? (uint64_t)d.n * a->n_head * nseg : 0;
 }
 
 /* An estimate of a prefill sequence's microseconds on this device, to choose
@@ -865,11 +855,9 @@ uint64_t prefill_rows(const janas_attn *a, const SeqDesc &d, const PrefillSplit 
    partials written and read back at 5 TB/s. The constants are a fit to 1042
    prompts of 80 .. 3000 tokens at 0 .. 8000 positions (16 shapes and cache
    types) with 1 .. 16 segments each, within 10 % of most. */
-double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, const PrefillSplit &sp,
-                        int exact)
+double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, bool halves, int exact,
+                        uint32_t nseg)
 {
-    const bool halves = sp.halves;
-    const uint32_t nseg = sp.nseg;
     const uint32_t tile = prefill_tile(a->hd, halves, exact);
     const uint32_t rows = prefill_block_rows(a->hd, halves, exact), R = d.n * a->group;
     const uint32_t nb = prefill_row_blocks(d.n, a->group, a->hd, halves, exact);
@@ -883,18 +871,7 @@ double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, const Pre
         const uint32_t lo = a->window && first + 1 > a->window ? first + 1 - a->window : 0;
         return hi / tile - lo / tile + 1;
     };
-    const uint64_t cus = a->cus;
-    const double merge_us =
-        nseg > 1 ? 3.0 + prefill_rows(a, d, sp, exact) * (a->hd + 2) * 8.0 / 5e6 : 0.0;
-    if (sp.blocks < nb) {
-        /* rounds of whole row blocks, then the split ones */
-        const uint64_t whole = (uint64_t)a->n_kv * (nb - sp.blocks);
-        const uint64_t rest = (uint64_t)a->n_kv * sp.blocks * nseg;
-        return (double)((whole + cus - 1) / cus) * (tiles(0) * tile_us + fixed_us) +
-               (double)((rest + cus - 1) / cus) *
-                   ((tiles(nb - sp.blocks) + nseg - 1) / nseg * tile_us + fixed_us) + merge_us;
-    }
-    const uint64_t per = (uint64_t)a->n_kv * nseg, N = nb * per;
+    const uint64_t per = (uint64_t)a->n_kv * nseg, N = nb * per, cus = a->cus;
     /* microseconds of the k-th longest workgroup */
     auto at = [&](uint64_t k) {
         return ((tiles(k / per) + nseg - 1) / nseg) * tile_us + fixed_us;
@@ -909,16 +886,14 @@ double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, const Pre
         const double even = (nb * a->n_kv * mean * tile_us + N * fixed_us) / cus;
         const double alike = at(N - 1) / longest;
         us = std::max(longest, alike * rounds * longest + (1 - alike) * even);
-        /* two rounds: the second's longest follows the first's shortest, its
-           shortest the longest of those that have one to follow. That alone
-           where the first's are alike (a window): they end together */
-        if (rounds == 2) {
-            const double pair =
-                std::max(longest, std::max(at(2 * cus - N) + at(N - 1), at(cus - 1) + at(cus)));
-            us = at(cus - 1) >= 0.9 * longest ? pair : (us + pair) / 2;
-        }
+        /* two rounds: the second's longest follows the shortest of the first
+           that has one to follow */
+        if (rounds == 2)
+            us = (us + std::max(longest, at(2 * cus - N) + at(N - 1))) / 2;
     }
-    return us + merge_us;
+    if (nseg > 1)
+        us += 3.0 + prefill_rows(a, d, nseg) * (a->hd + 2) * 8.0 / 5e6;
+    return us;
 }
 
 /* The split of a prefill sequence: prefill_halves' and prefill_segments',
@@ -926,11 +901,10 @@ double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, const Pre
    each compute unit a workgroup at least, and so leave a second round nearly
    empty where the row blocks do not divide the units (80 of them, 4 segments:
    320 workgroups for 256 units), and cut no segment below 6 tiles though a
-   short prefix has few; and one round and a half of equal workgroups (a long
-   prompt in a window) takes two: here the half round is split instead. Over the estimate's 1042 prompts the
-   choice takes 0.913 of the time (a 300-token int16 chunk at 8000 positions,
-   16 / 2 / 256, 245 -> 154 us; 80 tokens at 1024, 32 / 8 / 128 f16, 28 -> 19),
-   and 1.05 of it at worst; without the tenth it was 0.909, and 1.2 on some.
+   short prefix has few. Over the estimate's 1042 prompts the choice takes 0.913
+   of the time (a 300-token int16 chunk at 8000 positions, 16 / 2 / 256, 245 ->
+   154 us; 80 tokens at 1024, 32 / 8 / 128 f16, 28 -> 19), and 1.05 of it at
+   worst; without the tenth it was 0.909, and 1.2 on some.
    A sequence whose partials (and exact copy) would pass the allocation-free
    entry point's array keeps the first choice, and so do prompts of three
    rounds of workgroups, whose last one weighs little. base: the first choice
@@ -940,35 +914,25 @@ PrefillSplit prefill_split(const janas_attn *a, int kv, const SeqDesc &d, int ex
     PrefillSplit sp;
     sp.halves = !exact && prefill_halves(a, kv, d);
     sp.nseg = prefill_segments(a, d, sp.halves, exact);
-    const uint32_t blocks = prefill_row_blocks(d.n, a->group, a->hd, sp.halves, exact);
-    sp.blocks = sp.nseg > 1 ? blocks : 0;
-    if (base || (uint64_t)a->n_kv * blocks >= 3ull * a->cus)
+    if (base || (uint64_t)a->n_kv * prefill_row_blocks(d.n, a->group, a->hd, sp.halves, exact) >=
+                    3ull * a->cus)
         return sp;
     const uint64_t copy = 2ull * exact * a->n_kv * (d.end - d.c0 * kChunk) * a->hd * 2 + 512;
-    auto fits = [&](const PrefillSplit &x) {
-        return x.nseg < 2 || copy + 256 + prefill_rows(a, d, x, exact) * (a->hd + 2) *
-                                              sizeof(float) <= JANAS_ATTN_NOALLOC_BYTES;
-    };
-    double best = 0.9 * prefill_estimate(a, kv, d, PrefillSplit{sp.halves, sp.nseg, blocks}, exact);
-    auto offer = [&](const PrefillSplit &x, const PrefillSplit &as) {
-        const double us = prefill_estimate(a, kv, d, as, exact);
-        if (us < best && fits(x)) {
-            best = us;
-            sp = x;
-        }
-    };
+    double best = 0.9 * prefill_estimate(a, kv, d, sp.halves, exact, sp.nseg);
     for (int hv = !exact && prefill_halves_supported(kv, a->hd); hv >= 0; hv--) {
         const uint32_t tile = prefill_tile(a->hd, hv == 1, exact);
         const uint32_t first = a->window && d.pos0 + 1 > a->window ? d.pos0 + 1 - a->window : 0;
         const uint32_t nt = (d.end - 1) / tile - first / tile + 1;
-        const uint32_t nb = prefill_row_blocks(d.n, a->group, a->hd, hv == 1, exact);
-        for (uint32_t s = 1; s <= kMaxSegs && s <= nt; s++)
-            offer(PrefillSplit{hv == 1, s, s > 1 ? nb : 0}, PrefillSplit{hv == 1, s, nb});
-        /* whole rounds of row blocks as they are, the ones past them split */
-        const uint32_t round = a->cus / a->n_kv, rest = round && nb > round ? nb % round : 0;
-        if (rest && prefill_block_rows(a->hd, hv == 1, exact) % a->group == 0)
-            for (uint32_t s = 2; s <= 4; s++)
-                offer(PrefillSplit{hv == 1, s, rest}, PrefillSplit{hv == 1, s, rest});
+        for (uint32_t s = 1; s <= kMaxSegs && s <= nt; s++) {
+            if (s > 1 && copy + 256 + prefill_rows(a, d, s) * (a->hd + 2) * sizeof(float) >
+                             JANAS_ATTN_NOALLOC_BYTES)
+                break;
+            const double us = prefill_estimate(a, kv, d, hv == 1, exact, s);
+            if (us < best) {
+                best = us;
+                sp = PrefillSplit{hv == 1, s};
+            }
+        }
     }
     return sp;
 }
@@ -988,7 +952,7 @@ int prefill_splits(janas_attn *a, int kv, const janas_attn_seq *seqs, uint32_t n
             if (rc)
                 return rc;
             splits[i] = prefill_split(a, kv, d, exact, base);
-            rows += prefill_rows(a, d, splits[i], exact);
+            rows += prefill_rows(a, d, splits[i].nseg);
         }
         if (fixed) {
             if (reserve + rows * (a->hd + 2) * sizeof(float) + 256 <= JANAS_ATTN_NOALLOC_BYTES)
@@ -1036,18 +1000,15 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
                 d.wg0 = args.wg0s[m] = wg;
                 d.mg0 = args.mg0s[m] = mg;
                 d.nseg = splits[i].nseg;
-                d.rtiles = splits[i].blocks;
-                d.span = prefill_tokens(a, d, splits[i], exact);
                 d.part0 = 0;
-                uint64_t nwg = (uint64_t)a->n_kv *
-                               (prefill_row_blocks(d.n, a->group, a->hd, hv == 1, exact) +
-                                (uint64_t)d.rtiles * (d.nseg - 1));
+                uint64_t nwg = (uint64_t)a->n_kv * d.nseg *
+                               prefill_row_blocks(d.n, a->group, a->hd, hv == 1, exact);
                 uint64_t nmg = 0;
                 if (d.nseg > 1) {
                     /* partial rows from part0: (token, head) major, segment minor */
                     d.part0 = rows;
-                    rows += prefill_rows(a, d, splits[i], exact);
-                    nmg = pmerge_groups(d.span, a->n_head, a->hd);
+                    rows += (uint64_t)d.n * a->n_head * d.nseg;
+                    nmg = pmerge_groups(d.n, a->n_head, a->hd);
                 }
                 if (wg + nwg > 0x7FFFFFFFu || mg + nmg > 0x7FFFFFFFu)
                     return JANAS_ATTN_ERANGE;
@@ -1088,7 +1049,7 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
             /* Q8_K: the kernel's output or the segment merge wrote the
                blocks, or else a pass over the output does */
             for (uint32_t j = 0; j < m; j++) {
-                if (args.q8k_fused || args.seq[j].span == picked[j]->n)
+                if (args.q8k_fused || args.seq[j].nseg > 1)
                     continue;
                 rc = put_q8k(a, picked[j], 1, stream);
                 if (rc)

@@ -46,17 +46,13 @@ struct SeqDesc {
     const float *gate;     /* per GateMode, or null */
     const uint32_t *last;  /* [n] or null: token j sees up to pos0 + j */
     uint32_t cap, n, pos0, end; /* end: 1 + the last position any token sees */
-    uint32_t c0, span;     /* chunks c0 .. c0 + span - 1 are read; in a
-                              prefill launch, span: the first tokens whose
-                              row blocks are split (the segment merge's) */
+    uint32_t c0, span;     /* chunks c0 .. c0 + span - 1 are read */
     uint32_t rtiles;       /* workgroups along the query rows (rows = n x
-                              group): of split_tile_rows(hd) x mt rows; in a
-                              prefill launch, the row blocks of a KV head
-                              that are split, from row 0 on */
+                              group): of split_tile_rows(hd) x mt rows */
     uint32_t wg0;          /* first workgroup of the split launch */
     uint32_t mg0;          /* first workgroup of the merge launch */
-    uint32_t nseg;         /* prefill: key segments a split row block has
-                              (one that is not writes its output) */
+    uint32_t nseg;         /* prefill: key segments a row block is split
+                              into (1: none, the output is written directly) */
     uint64_t part0;        /* first partial row (of m, l and hd values) */
     void *q8k;             /* the output also as Q8_K blocks, or null */
 };

@@ -268,21 +268,18 @@ __device__ __forceinline__ PBlock block_of(const PrefillArgs &A)
     P.sq = &A.seq[si];
     const SeqDesc &sq = *P.sq;
     /* the descriptor fields the block starts from in one round trip */
-    asm volatile("" ::"s"(sq.n), "s"(sq.nseg), "s"(sq.rtiles), "s"(sq.wg0), "s"(sq.pos0), "s"(sq.end),
+    asm volatile("" ::"s"(sq.n), "s"(sq.nseg), "s"(sq.wg0), "s"(sq.pos0), "s"(sq.end),
                  "s"(sq.cap), "s"(sq.last), "s"(sq.q), "s"(sq.k), "s"(sq.v));
     const uint32_t G = A.group;
     const uint32_t R = sq.n * G;
     const uint32_t nrb = (R + kPBlock - 1) / kPBlock;
-    /* a KV head's workgroups: row blocks, the longest rows first, the first
-       ones whole and the last sq.rtiles of them in nseg key segments each */
-    const uint32_t nsplit = sq.rtiles, whole = nrb - nsplit;
-    const uint32_t per = whole + nsplit * sq.nseg;
+    /* a KV head's workgroups: row blocks, the longest rows first, each
+       split into nseg key segments */
+    const uint32_t nseg = sq.nseg;
     const uint32_t local = id - sq.wg0;
-    const uint32_t kvh = local / per;
-    const uint32_t rem = local % per;
-    const bool cut = rem >= whole;
-    const uint32_t nseg = cut ? sq.nseg : 1, x = cut ? rem - whole : rem;
-    const uint32_t rb = (cut ? nsplit : nrb) - 1 - x / nseg;
+    const uint32_t kvh = local / (nrb * nseg);
+    const uint32_t rem = local % (nrb * nseg);
+    const uint32_t rb = nrb - 1 - rem / nseg;
     const uint32_t r0 = rb * kPBlock;
 
     /* the block's rows see [lo(first token), hi(last token)] */
@@ -297,7 +294,7 @@ __device__ __forceinline__ PBlock block_of(const PrefillArgs &A)
        empty one (a block with fewer tiles than segments) runs its first
        tile with every row masked, which leaves the neutral partial
        (m = -inf, no weight) - no branch around the tile loop */
-    P.seg = x % nseg;
+    P.seg = rem % nseg;
     P.nseg = nseg;
     bool empty = false;
     if (nseg > 1) {
@@ -1757,7 +1754,7 @@ __global__ __launch_bounds__(kPMergeThreads) void pmerge_kernel(const PrefillArg
     const uint32_t row = (uint32_t)(pair / c4), col = (uint32_t)(pair % c4) * 4;
     /* past the sequence's rows: whole waves, since with Q8_K its outputs
        are whole blocks of 64 pairs */
-    if (row >= sq.span * A.n_head)
+    if (row >= sq.n * A.n_head)
         return;
     const uint32_t j = row / A.n_head, h = row % A.n_head;
     const size_t pr0 = sq.part0 + (size_t)row * nseg;
