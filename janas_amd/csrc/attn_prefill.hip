@@ -1024,13 +1024,14 @@ __global__ __launch_bounds__(PCfg<D>::W * 64) void prefill_dma_kernel(const Pref
  * f16 planes whose sum is the cached number exactly (int8: one plane; int16:
  * the nearest f16, and what is left, at most 8), and the query and the
  * weights as two f16 planes each (x = hi + lo, 22 significant bits), so each
- * product is exact in the matrix core and summed in f32. Over int16 three of
- * the four plane products are made: both low planes are at most 2^-11 of
- * their numbers, so low times low is at most 2^-22 of the product, as much as
- * the query's and the weights' two planes leave of them (x & 255 as the low
- * plane is no such part of a small x: low times low was made). A 3001-token prompt at 16 / 2 / 256 in a window of 1024 265
- * -> 231 us, 4096 tokens at 32 / 8 / 128 523 -> 444 us, the error against 64
- * bits 9.4e-7 -> 8.7e-7 and 8.6e-7 -> 8.0e-7. The scales stay f32:
+ * product is exact in the matrix core and summed in f32. Over int16 all four
+ * plane products are made: low times low is up to 2^-22 of a product, four
+ * times what the rounding of an f32 sum leaves of it. (Without it 4096 tokens
+ * at 32 / 8 / 128 in a window of 1024 took 242 us for 278, and rows whose low
+ * products have one sign missed them.) The nearest f16 and the rest as planes
+ * leave smaller second products than 256 (x >> 8) and x & 255, so smaller
+ * roundings of their sums: the error of a 3001-token prompt at 16 / 2 / 256 in
+ * a window of 1024 against 64 bits is 8.7e-7 for 9.6e-7. The scales stay f32:
  *   score   s = (sum_i q'_i k_i) * ks[p] * 2^-e,  q' = q * scale * log2(e) * 2^e
  *           (e puts the row's largest |q'| in [2^13, 2^14): neither plane
  *           loses bits to f16's range)
@@ -1150,8 +1151,7 @@ __device__ __forceinline__ float load_query_x(const PrefillArgs &A, const PBlock
 
 /*
  * One key tile of the exact kernel for the lane's row: the tile pass of
- * tile_pass with planes (both of the query's and weights' with plane 0, the
- * high one with plane 1). kop(s, b, p): plane p of the score operand (K rows
+ * tile_pass with planes. kop(s, b, p): plane p of the score operand (K rows
  * 32 b + l % 32, columns 16 s + 8 (l / 32) ..); vop(ks, c, p): plane p of the
  * value operand; sop(which, b, j): the key (which 0) or value (1) scales of
  * positions 32 b + 8 j + 4 (l / 32) + 0..3 of the tile; lop(s): the loads
@@ -1196,8 +1196,7 @@ __device__ __forceinline__ void tile_pass_x(uint32_t p0, const PBlock &P, const 
 #pragma unroll
             for (int p = 0; p < NP; p++) {
                 sacc[b] = mfma(ka[s & 1][b][p], qh[s], sacc[b]);
-                if (p == 0)
-                    sacc[b] = mfma(ka[s & 1][b][p], ql[s], sacc[b]);
+                sacc[b] = mfma(ka[s & 1][b][p], ql[s], sacc[b]);
             }
     }
     __builtin_amdgcn_sched_group_barrier(0x100, kNPB * NP, 0);
@@ -1206,7 +1205,7 @@ __device__ __forceinline__ void tile_pass_x(uint32_t p0, const PBlock &P, const 
         sgb_vmem(xloads_at<NL, KS>(s));
         if (s + 1 < KS)
             __builtin_amdgcn_sched_group_barrier(0x100, kNPB * NP, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, kNPB * (NP + 1), 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * kNPB * NP, 0);
     }
 
     /* the key scales, the query's 2^-e, and the weights' 2^kB less the
@@ -1330,8 +1329,7 @@ __device__ __forceinline__ void tile_pass_x(uint32_t p0, const PBlock &P, const 
 #pragma unroll
             for (int p = 0; p < NP; p++) {
                 o[c] = mfma(va[ks & 1][c][p], ph[ks & 1], o[c]);
-                if (p == 0)
-                    o[c] = mfma(va[ks & 1][c][p], pl[ks & 1], o[c]);
+                o[c] = mfma(va[ks & 1][c][p], pl[ks & 1], o[c]);
             }
     }
     lsum += ls;

@@ -431,31 +431,71 @@ def test_prefill_quantized_cache(gpu, wide, geom):
     assert within(err, quantized_bar(hd), "vs oracle")
 
 
+def low_plane(x):
+    """x - f16(x): what is left of numbers past their nearest f16"""
+    x = np.asarray(x, np.float64)
+    return x - x.astype(np.float16).astype(np.float64)
+
+
 @pytest.mark.parametrize("hd", [64, 128, 256])
-def test_prefill_int16_low_planes(gpu, hd):
-    """int16 numbers whose planes f16(x) and x - f16(x) are the largest (8 off,
-    the ends of the range) under queries whose low plane is the largest and of
-    one sign, so that what the products leave out - low plane times low plane,
-    at most 2^-24 of |q x| each - adds up: scores of sum |q x| scale <= 16
-    move by 2^-20, outputs of magnitude up to 1 by 2^-19 and the f32 sums'
-    rounding, inside the FLOAT bar."""
+@pytest.mark.parametrize("part", ["scores", "values"])
+def test_prefill_int16_low_planes(gpu, part, hd):
+    """int16 caches: the low plane of an integer (what is left of it past its
+    nearest f16) times the low plane of the query or of a weight counts.
+
+    Integers 16392 and 16408 are ties of f16, low planes +8 and -8. The
+    products come in pairs that nearly cancel, with low plane times low plane
+    of one sign: 2^-22 of the sum of magnitudes, which a kernel without that
+    product misses (asserted below), while f32 sums, whose partial sums stay
+    within one product of magnitude M / N of N, keep the sum to N 2^-24 M / N
+    = 2^-24 M even if every addition rounds the same way.
+
+    scores: M is 1024 nats over a row, the positions of two kinds with their
+    low products of either sign: the softmax between them (weights p and 1 - p,
+    values 1 and -1) moves by 2 p (1 - p) times twice that. values: equal
+    weights, M = 1."""
     h, kvh, n, cap = 4, 2, 130, 300
     rng = np.random.default_rng(hd)
-    pick = np.array([32767, 32760, 32744, 20488, 16392, -32768, -16392, 8196, 4098], np.int16)
-    k, v = (pick[rng.integers(0, len(pick), (kvh, cap, hd))] for _ in range(2))
-    ks = np.full((kvh, cap), 1.0 / 32768, np.float32)
-    sign = np.where(rng.random((n, h, hd)) < 0.5, -1.0, 1.0)
-    q = (sign * (1.0 + 2.0 ** -11 - 2.0 ** -22)).astype(np.float32)
+    f = np.float32(1.0 / np.sqrt(np.float32(hd))) * np.float32(np.log2(np.e))
+    if part == "scores":
+        t = 8196 - 2.0 ** -8              # the query as the products take it
+        sign = np.where(rng.random((kvh, hd)) < 0.5, -1, 1)
+        q = np.repeat(sign, h // kvh, 0)[None].repeat(n, 0) * np.float32(t / f)
+        kind = rng.random((kvh, cap)) < 0.5
+        pair = np.tile([1, -1], hd // 2)  # a number's sign against the query's
+        up = np.where(pair > 0, 16392, -16408)      # low planes +8, with the query
+        down = np.where(pair > 0, 16408, -16392)    # -8
+        k = (np.where(kind[..., None], up, down) * sign[:, None]).astype(np.int16)
+        v = np.where(kind[..., None], 32767, -32767).repeat(hd, 2).astype(np.int16)
+        big = 1024.0
+        ks = np.full((kvh, cap), big * np.log2(np.e) / (hd * t * 16400), np.float32)
+        vs = np.full((kvh, cap), 1.0 / 32767, np.float32)
+        missed = (low_plane(q[0, ::h // kvh] * f)[:, None] * low_plane(k)).sum(2) * ks * np.log(2)
+        assert (np.abs(missed) > 0.99 * big * 2.0 ** -22).all()
+        assert (np.sign(missed) == np.where(kind, 1, -1)).all()
+        bar = 2 * 0.25 * 2 * big * 2.0 ** -24
+    else:
+        q = np.zeros((n, h, hd))
+        k = rng.integers(-32767, 32768, (kvh, cap, hd)).astype(np.int16)
+        ks = np.full((kvh, cap), 1.0 / 32768, np.float32)
+        pair = np.where(np.arange(cap) % 2 == 0, 16392, -16408)
+        v = pair[None, :, None].repeat(kvh, 0).repeat(hd, 2).astype(np.int16)
+        vs = np.full((kvh, cap), 2.0 ** -14 * (1 + 2.0 ** -11 - 2.0 ** -20), np.float32)
+        missed = low_plane(vs * 2.0 ** 14) * 2.0 ** -14 * low_plane(v[..., 0])
+        assert (missed > 0.99 * 2.0 ** -22).all()
+        # (and the division by the sum of the weights, and the output's rounding)
+        bar = 2.0 ** -24 + 2.0 ** -24 * 8 / 16400 * 4
+    q = q.astype(np.float32)
     out = torch.full((n, h, hd), float("nan"), device=gpu)
     with Attention(h, kvh, hd, cap) as a:
         a.run_dev(janas_amd.KV_I16, [dict(
             k=to_dev(k, gpu), v=to_dev(v, gpu), ks=to_dev(ks, gpu),
-            vs=to_dev(ks, gpu), q=to_dev(q, gpu), out=out, cap=cap, n=n,
+            vs=to_dev(vs, gpu), q=to_dev(q, gpu), out=out, cap=cap, n=n,
             pos0=cap - n)], path="prefill")
         torch.cuda.synchronize()
-    ref = orc.exact(q, k, v, ks, ks, n_head=h, n_kv=kvh, hd=hd, pos0=cap - n,
+    ref = orc.exact(q, k, v, ks, vs, n_head=h, n_kv=kvh, hd=hd, pos0=cap - n,
                     kv=janas_amd.KV_I16)
-    assert within(abs_err(out.cpu().numpy(), ref), TOL_FLOAT_ABS, "vs exact")
+    assert within(abs_err(out.cpu().numpy(), ref), bar, "vs exact")
 
 
 @pytest.mark.parametrize("hd", [128, 64, 256])
