@@ -14,9 +14,7 @@
 #include <sys/stat.h>
 
 #include <algorithm>
-#include <memory>
 #include <mutex>
-#include <new>
 #include <string>
 #include <vector>
 
@@ -781,14 +779,13 @@ void choose_way_dev(janas_attn *a, int kv, const janas_attn_seq *seqs, uint32_t 
     a->scores = int16 ? JANAS_ATTN_INT16 : JANAS_ATTN_FLOAT;
 }
 
-/* Key segments for a prefill sequence whose row blocks alone would leave
-   compute units idle (a short prompt, a chunk of a long one): enough to
+/* The most key segments of a prefill sequence whose row blocks alone would
+   leave compute units idle (a short prompt, a chunk of a long one): enough to
    give each unit a workgroup, at least kSegTiles key tiles each (twice as
-   many with the halves' tiles, which two groups share). It depends on the
-   sequence alone, so a sequence's result is the same in any launch. */
+   many with the halves' tiles, which two groups share). */
 constexpr uint32_t kSegTiles = 6;
 
-uint32_t prefill_segments(const janas_attn *a, const SeqDesc &d, bool halves, int exact)
+uint32_t prefill_most_segments(const janas_attn *a, const SeqDesc &d, bool halves, int exact)
 {
     const uint64_t blocks =
         (uint64_t)a->n_kv * prefill_row_blocks(d.n, a->group, a->hd, halves, exact);
@@ -831,29 +828,17 @@ bool prefill_halves(const janas_attn *a, int kv, const SeqDesc &d)
 {
     if (!prefill_halves_supported(kv, a->hd))
         return false;
-    const uint64_t wg = (uint64_t)a->n_kv * prefill_segments(a, d, false, 0) *
+    const uint64_t wg = (uint64_t)a->n_kv * prefill_most_segments(a, d, false, 0) *
                         prefill_row_blocks(d.n, a->group, a->hd, false);
     return wg < a->cus;
 }
 
-/* How a prefill sequence is split: the kernel and the key segments. */
-struct PrefillSplit {
-    bool halves;
-    uint32_t nseg;
-};
-
-/* partial rows of a split sequence */
-uint64_t prefill_rows(const janas_attn *a, const SeqDesc &d, uint32_t nseg)
-{
-    return nseg > 1 ? (uint64_t)d.n * a->n_head * nseg : 0;
-}
-
-/* An estimate of a prefill sequence's microseconds on this device, to choose
-   between splits with: its workgroups take the compute units in rounds,
-   longest rows first, one workgroup a unit (their LDS or registers fill it),
-   a workgroup 4 us and its tiles' time; a split adds a merge of 3 us and the
-   partials written and read back at 5 TB/s. The constants are a fit to 1042
-   prompts of 80 .. 3000 tokens at 0 .. 8000 positions (16 shapes and cache
+/* An estimate of a prefill sequence's microseconds on this device in nseg key
+   segments, to choose between them with: its workgroups take the compute units
+   in rounds, longest rows first, one workgroup a unit (their LDS or registers
+   fill it), a workgroup 4 us and its tiles' time; segments add a merge of 3 us
+   and the partials written and read back at 5 TB/s. The constants are a fit to
+   1042 prompts of 80 .. 3000 tokens at 0 .. 8000 positions (16 shapes and cache
    types) with 1 .. 16 segments each, within 10 % of most. */
 double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, bool halves, int exact,
                         uint32_t nseg)
@@ -892,80 +877,40 @@ double prefill_estimate(const janas_attn *a, int kv, const SeqDesc &d, bool halv
             us = (us + std::max(longest, at(2 * cus - N) + at(N - 1))) / 2;
     }
     if (nseg > 1)
-        us += 3.0 + prefill_rows(a, d, nseg) * (a->hd + 2) * 8.0 / 5e6;
+        us += 3.0 + (double)d.n * a->n_head * nseg * (a->hd + 2) * 8.0 / 5e6;
     return us;
 }
 
-/* The split of a prefill sequence: prefill_halves' and prefill_segments',
-   unless the estimate of another is shorter by over a tenth. Those two give
-   each compute unit a workgroup at least, and so leave a second round nearly
-   empty where the row blocks do not divide the units (80 of them, 4 segments:
-   320 workgroups for 256 units), and cut no segment below 6 tiles though a
-   short prefix has few. Over the estimate's 1042 prompts the choice takes 0.913
-   of the time (a 300-token int16 chunk at 8000 positions, 16 / 2 / 256, 245 ->
-   154 us; 80 tokens at 1024, 32 / 8 / 128 f16, 28 -> 19), and 1.05 of it at
-   worst; without the tenth it was 0.909, and 1.2 on some.
-   A sequence whose partials (and exact copy) would pass the allocation-free
-   entry point's array keeps the first choice, and so do prompts of three
-   rounds of workgroups, whose last one weighs little. base: the first choice
-   alone. It depends on the sequence and the device alone. */
-PrefillSplit prefill_split(const janas_attn *a, int kv, const SeqDesc &d, int exact, bool base)
+/* A prefill sequence's key segments: the most, or fewer where their estimate is
+   shorter by a fifth. The most leave a second round of workgroups nearly empty
+   where the row blocks do not divide the units (84 of them in 4 segments are
+   336 workgroups for 256 units, in 3 one round: 672 int16 tokens at 3202
+   positions, 16 / 2 / 256, 222 -> 171 us). A fifth, since the estimate takes
+   the second round for longer than it is by up to that; three tenths at head
+   sizes up to 64, where a unit holds two workgroups and it is shorter still.
+   Over 90 prompts that take fewer a call takes 0.78 of the time (1.03 at worst),
+   and calls of 2, 4 and 8 of each 0.84 - 0.85 (1.11 at worst).
+   Never more than the most: the segments past it that make a prompt shorter
+   which has the device to itself (80 tokens at 1024 positions, 32 / 8 / 128
+   f16, 25 -> 22 us) cost several of them in one call up to 2.6 times the time
+   (16: 56 -> 145 us), and the partials of calls that had none.
+   The choice depends on the sequence and the device alone, so a sequence's
+   result is the same in any launch. */
+uint32_t prefill_segments(const janas_attn *a, int kv, const SeqDesc &d, bool halves, int exact)
 {
-    PrefillSplit sp;
-    sp.halves = !exact && prefill_halves(a, kv, d);
-    sp.nseg = prefill_segments(a, d, sp.halves, exact);
-    if (base || (uint64_t)a->n_kv * prefill_row_blocks(d.n, a->group, a->hd, sp.halves, exact) >=
-                    3ull * a->cus)
-        return sp;
-    const uint64_t copy = 2ull * exact * a->n_kv * (d.end - d.c0 * kChunk) * a->hd * 2 + 512;
-    double best = 0.9 * prefill_estimate(a, kv, d, sp.halves, exact, sp.nseg);
-    for (int hv = !exact && prefill_halves_supported(kv, a->hd); hv >= 0; hv--) {
-        const uint32_t tile = prefill_tile(a->hd, hv == 1, exact);
-        const uint32_t first = a->window && d.pos0 + 1 > a->window ? d.pos0 + 1 - a->window : 0;
-        const uint32_t nt = (d.end - 1) / tile - first / tile + 1;
-        for (uint32_t s = 1; s <= kMaxSegs && s <= nt; s++) {
-            if (s > 1 && copy + 256 + prefill_rows(a, d, s) * (a->hd + 2) * sizeof(float) >
-                             JANAS_ATTN_NOALLOC_BYTES)
-                break;
-            const double us = prefill_estimate(a, kv, d, hv == 1, exact, s);
-            if (us < best) {
-                best = us;
-                sp = PrefillSplit{hv == 1, s};
-            }
+    const uint32_t most = prefill_most_segments(a, d, halves, exact);
+    if (most < 2)
+        return 1;
+    uint32_t nseg = most;
+    double best = (a->hd > 64 ? 0.8 : 0.7) * prefill_estimate(a, kv, d, halves, exact, most);
+    for (uint32_t s = 1; s < most; s++) {
+        const double us = prefill_estimate(a, kv, d, halves, exact, s);
+        if (us < best) {
+            best = us;
+            nseg = s;
         }
     }
-    return sp;
-}
-
-/* The splits of a call's sequences: the first choices alone where the partials
-   would otherwise pass the fixed array, or need more rows than the instance
-   has while the stream is captured. */
-int prefill_splits(janas_attn *a, int kv, const janas_attn_seq *seqs, uint32_t n_seqs, int exact,
-                   hipStream_t stream, bool fixed, uint64_t reserve,
-                   PrefillSplit *splits)
-{
-    for (int base = 0; base < 2; base++) {
-        uint64_t rows = 0;
-        for (uint32_t i = 0; i < n_seqs; i++) {
-            SeqDesc d;
-            int rc = describe(a, kv, seqs[i], d);
-            if (rc)
-                return rc;
-            splits[i] = prefill_split(a, kv, d, exact, base);
-            rows += prefill_rows(a, d, splits[i].nseg);
-        }
-        if (fixed) {
-            if (reserve + rows * (a->hd + 2) * sizeof(float) + 256 <= JANAS_ATTN_NOALLOC_BYTES)
-                break;
-        } else {
-            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-            if (rows > a->part_rows && hipStreamIsCapturing(stream, &cs) != hipSuccess)
-                (void)hipGetLastError();
-            if (cs == hipStreamCaptureStatusNone)
-                break;
-        }
-    }
-    return JANAS_ATTN_OK;
+    return nseg;
 }
 
 /* The sequences in launches of up to kMaxSeqs, those that take the
@@ -976,14 +921,7 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
                        const janas_attn_seq *seqs, uint32_t n_seqs, hipStream_t stream,
                        bool fixed, int exact = 0, uint64_t reserve = 0)
 {
-    /* (no exception may leave the C entry point) */
-    std::unique_ptr<PrefillSplit[]> splits(new (std::nothrow) PrefillSplit[n_seqs]);
-    if (!splits)
-        return JANAS_ATTN_ENOMEM;
-    int rc = prefill_splits(a, kv, seqs, n_seqs, exact, stream, fixed, reserve, splits.get());
-    if (rc)
-        return rc;
-    for (int hv = !exact && prefill_halves_supported(kv, a->hd); hv >= 0; hv--) {
+    for (int hv = 1; hv >= 0; hv--) {
         for (uint32_t i = 0; i < n_seqs;) {
             PrefillArgs args;
             memset(&args, 0, sizeof args);
@@ -992,14 +930,14 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
             uint64_t rows = 0;
             for (; i < n_seqs && m < kMaxSeqs; i++) {
                 SeqDesc &d = args.seq[m];
-                rc = describe(a, kv, seqs[i], d);
+                int rc = describe(a, kv, seqs[i], d);
                 if (rc)
                     return rc;
-                if (splits[i].halves != (hv == 1))
+                if ((!exact && prefill_halves(a, kv, d)) != (hv == 1))
                     continue;
                 d.wg0 = args.wg0s[m] = wg;
                 d.mg0 = args.mg0s[m] = mg;
-                d.nseg = splits[i].nseg;
+                d.nseg = prefill_segments(a, kv, d, hv == 1, exact);
                 d.part0 = 0;
                 uint64_t nwg = (uint64_t)a->n_kv * d.nseg *
                                prefill_row_blocks(d.n, a->group, a->hd, hv == 1, exact);
@@ -1020,7 +958,7 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
                 break;
             Parts pt{nullptr, nullptr, fixed};
             if (rows) {
-                rc = get_parts(a, rows, stream, fixed, pt, reserve);
+                int rc = get_parts(a, rows, stream, fixed, pt, reserve);
                 if (rc)
                     return rc;
             }
@@ -1051,7 +989,7 @@ int run_prefill_launch(janas_attn *a, int kv, int gate_mode,
             for (uint32_t j = 0; j < m; j++) {
                 if (args.q8k_fused || args.seq[j].nseg > 1)
                     continue;
-                rc = put_q8k(a, picked[j], 1, stream);
+                int rc = put_q8k(a, picked[j], 1, stream);
                 if (rc)
                     return rc;
             }

@@ -84,7 +84,7 @@ def fill(host, geom, kv, window, n, pos0):
 
 # prompts of more than one round of workgroups, of like length in a window
 WINDOWED = [((16, 2, 256), I16, 1024, 3001, 0), ((16, 2, 256), F16, 700, 3001, 0),
-            ((8, 2, 256), I8, 400, 4333, 900)]
+            ((8, 2, 256), I8, 400, 4333, 900), ((32, 8, 128), F16, 512, 4432, 4000)]
 
 
 @pytest.mark.parametrize("geom,kv,window,n,pos0", WINDOWED)
@@ -100,3 +100,64 @@ def test_prompts_that_fill_the_device_use_no_partials(host, geom, kv, window, n,
         assert got.rc == 0
         assert got.prompts() == [(hv, 1, False)] * m
         assert got.workgroups() == m * blocks
+
+
+# short prompts, chunks, and prompts of less than a round of workgroups
+PROMPTS = [((32, 8, 128), F16, 0, 80, 1024), ((12, 4, 64), F16, 1024, 1000, 0),
+           ((16, 2, 256), F16, 0, 300, 256), ((32, 8, 128), I8, 0, 150, 512),
+           ((32, 4, 128), I8, 0, 300, 512), ((16, 2, 256), I16, 0, 200, 0),
+           ((32, 8, 128), I8, 0, 80, 1000), ((16, 2, 256), I16, 0, 300, 8000),
+           ((12, 4, 64), F16, 0, 1147, 0), ((12, 4, 64), I16, 0, 900, 300),
+           ((32, 8, 128), F16, 0, 512, 2048), ((16, 2, 512), F16, 0, 99, 7452),
+           ((16, 2, 512), I16, 1024, 399, 972), ((32, 8, 128), F16, 0, 1432, 0),
+           ((12, 4, 64), F16, 1024, 3500, 0), ((32, 8, 128), F16, 512, 1432, 4000)] + WINDOWED
+
+
+@pytest.mark.parametrize("geom,kv,window,n,pos0", PROMPTS)
+def test_segments_follow_the_sequence_and_stay_few(host, geom, kv, window, n, pos0):
+    """The kernel that fills the device, and no more segments than fill it: in a
+    call alone, in one of 2 to 40 prompts, beside a longer one, through the entry
+    point without allocation (where a copy and partials fit it), after calls that
+    grew the instance, and captured - always the same."""
+    hv, most, blocks = fill(host, geom, kv, window, n, pos0)
+    h, n_kv, hd = geom
+    new = f"new {h} {n_kv} {hd} {window} 256"
+    one = f" {n} {pos0}"
+    lines = [new, f"call dev {kv} 0 0{one}", f"call noalloc {kv} 0 0{one}",
+             f"call dev {kv} 0 0 4000 3000{one}", f"call dev {kv} 0 1{one}"]
+    alone, noalloc, beside, captured = (Call(w) for w in host(lines)[1:])
+    assert alone.rc == 0
+    (got,) = alone.prompts()
+    assert got[0] == hv and 1 <= got[1] <= most and got[2] == (got[1] > 1)
+    assert alone.workgroups() == blocks * got[1]
+    assert noalloc.rc in (0, janas_amd.ERANGE)
+    if noalloc.rc == 0:
+        assert noalloc.prompts() == [got]
+    assert got[:2] in [x[:2] for x in beside.prompts()]
+    assert captured.rc == 0 and captured.refused == 0
+    assert captured.prompts() == [got]
+    for m in (2, 3, 8, 16, 40):
+        many = Call(host([new, f"call dev {kv} 0 0" + one * m])[1])
+        assert many.prompts() == [got] * m
+        assert many.workgroups() == m * blocks * got[1]
+
+
+@pytest.mark.parametrize("geom,kv,window,n,pos0", [c for c in PROMPTS if c[1] == F16])
+def test_prompts_without_segments_leave_the_instance_alone(host, geom, kv, window, n, pos0):
+    """An f16 prompt that segments cannot make fill the device any better uses no
+    memory of the instance: nothing is allocated at its first call, a captured
+    one holds none that a later call could free, and after work of the instance
+    on another stream it neither waits for it nor is refused under capture."""
+    _, most, _ = fill(host, geom, kv, window, n, pos0)
+    if most > 1:
+        pytest.skip("a prompt that takes segments")
+    h, n_kv, hd = geom
+    one = f" {n} {pos0}"
+    # (a decode of 300 positions leaves partials on stream 0)
+    for captured in (0, 1):
+        new, decode, call = host([f"new {h} {n_kv} {hd} {window} 256", f"call dev {kv} 0 0 1 299",
+                                  f"call dev {kv} 1 {captured}{one}"])
+        got = Call(call)
+        assert got.rc == 0
+        assert (got.allocs, got.frees, got.refused, got.waits) == (0, 0, 0, 0)
+        assert all(not parts for _, _, parts, _, _ in got.launches)
