@@ -56,7 +56,7 @@ struct janas_attn {
     int dev;
     uint32_t cus;         /* compute units of the device */
     hipStream_t stream;
-    /* partials: part_rows rows of hd values, then of (m, l), one block */
+    /* partials: part_rows rows of (m, l) and of hd values */
     float *part_ml, *part_acc;
     uint64_t part_rows;
     /* the stream that last used the partials: a call on another stream
@@ -257,12 +257,11 @@ int part_sync(janas_attn *a, hipStream_t stream)
 
 void free_part(janas_attn *a)
 {
+    (void)hipFree(a->part_ml);
     (void)hipFree(a->part_acc);
     a->part_ml = a->part_acc = nullptr;
     a->part_rows = 0;
 }
-
-constexpr uint64_t kPage = 2u << 20;
 
 int ensure_part(janas_attn *a, uint64_t rows, hipStream_t stream)
 {
@@ -270,7 +269,7 @@ int ensure_part(janas_attn *a, uint64_t rows, hipStream_t stream)
         return JANAS_ATTN_OK;
     /* the stream that used them last, and this one, may still read the
        old ones */
-    if (a->part_acc) {
+    if (a->part_ml || a->part_acc) {
         hipError_t e = hipStreamSynchronize(stream);
         if (e == hipSuccess && a->part_stream && a->part_stream != stream)
             e = hipStreamSynchronize(a->part_stream);
@@ -278,25 +277,15 @@ int ensure_part(janas_attn *a, uint64_t rows, hipStream_t stream)
             return hip_err(e, "synchronize");
         free_part(a);
     }
-    /* whole pages of 2 MiB, none of the tail in small ones: a ragged decode of
-       8 sequences 31.7 - 31.8 us for 31.9 - 32.2 */
-    const uint64_t bytes = (rows * (a->hd + 2) * sizeof(float) + kPage - 1) / kPage * kPage;
-    if (hipMalloc(&a->part_acc, bytes) != hipSuccess) {
+    if (hipMalloc(&a->part_ml, rows * 2 * sizeof(float)) != hipSuccess ||
+        hipMalloc(&a->part_acc, rows * a->hd * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
-        a->part_acc = nullptr;
+        free_part(a);
         return JANAS_ATTN_ENOMEM;
     }
-    /* (hd is a multiple of 8: the pairs stay aligned) */
-    a->part_ml = a->part_acc + rows * a->hd;
     a->part_rows = rows;
     return JANAS_ATTN_OK;
 }
-
-/* an instance's partials from its creation on, at least: a prompt of some
-   hundred tokens in a few key segments needs no more, so its first call does
-   not free and allocate (64 us; creating an instance that needs less takes 30
-   - 50 us more) */
-constexpr uint64_t kPartBytes = 16u << 20;
 
 /* Where a call's partials live: the instance's (grown as needed, ordered
    across streams), or the device's fixed array of the allocation-free
@@ -1215,11 +1204,10 @@ extern "C" struct janas_attn *janas_attn_create(uint32_t n_head,
         return nullptr;
     }
     /* the partials of a full janas_attn_run block, as the reference
-       allocates them (attention.c:1013), and at least kPartBytes */
+       allocates them (attention.c:1013) */
     uint32_t chunks = (n_ctx + kChunk - 1) / kChunk;
     uint64_t rows = (uint64_t)n_head_kv * (chunks ? chunks : 1) *
                     JANAS_ATTN_MAX_BLOCK * a->group;
-    rows = std::max<uint64_t>(rows, kPartBytes / ((head_dim + 2) * sizeof(float)));
     if (ensure_part(a, rows, a->stream) != JANAS_ATTN_OK) {
         janas_attn_destroy(a);
         return nullptr;

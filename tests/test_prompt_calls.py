@@ -161,3 +161,14 @@ def test_prompts_without_segments_leave_the_instance_alone(host, geom, kv, windo
         assert got.rc == 0
         assert (got.allocs, got.frees, got.refused, got.waits) == (0, 0, 0, 0)
         assert all(not parts for _, _, parts, _, _ in got.launches)
+
+
+@pytest.mark.parametrize("geom,n_ctx", [((32, 8, 128), 256), ((12, 4, 64), 600),
+                                        ((16, 2, 512), 32768), ((8, 8, 8), 0)])
+def test_an_instance_holds_a_blocks_partials(host, geom, n_ctx):
+    """What janas_attn_part_bytes says from the creation on (at least a chunk's),
+    in one allocation for the pairs and one for the values."""
+    h, n_kv, hd = geom
+    rows, allocs = (int(x) for x in host([f"new {h} {n_kv} {hd} 0 {n_ctx}"])[0])
+    assert rows * (hd + 2) * 4 == janas_amd.part_bytes(h, n_kv, hd, max(n_ctx, 1))
+    assert allocs == 2
