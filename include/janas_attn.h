@@ -270,7 +270,12 @@ int janas_attn_run_dev_noalloc(struct janas_attn *a, int kv_type, int gate_mode,
 
 /* For measurement: the split-KV path's kernels one at a time - kernels 1
    the split kernel alone (partials only), 2 the merge alone (over the
-   partials a previous call left), 3 both (janas_attn_run_dev_split). */
+   partials a previous call left), 3 both, one after the other.
+   janas_attn_run_dev and _split launch the split kernel alone, which then
+   writes the outputs and no partials, where every sequence of a launch sees
+   one chunk at a head size up to 256 and none asks for Q8_K blocks: 3 gives
+   the same bits in two launches, and 2 after such a call makes the partials
+   first. */
 int janas_attn_run_dev_kernels(struct janas_attn *a, int kv_type,
                                int gate_mode,
                                const struct janas_attn_seq *seqs,
@@ -282,8 +287,9 @@ const char *janas_attn_strerror(int err);
 /*
  * Kernel timing for measurement: while on, every launch of the instance is
  * bracketed by HIP events on its stream; janas_attn_prof_read returns, per
- * kernel (0 split, 1 merge, 2 prefill), the launches and their summed
- * milliseconds (synchronizing the stream), and zeroes them.
+ * kernel (0 split, 1 merge - none where the split kernel writes the outputs -,
+ * 2 prefill), the launches and their summed milliseconds (synchronizing the
+ * stream), and zeroes them.
  */
 void janas_attn_prof_enable(struct janas_attn *a, int on);
 int janas_attn_prof_read(struct janas_attn *a, uint32_t counts[3],

@@ -59,6 +59,8 @@ struct janas_attn {
     /* partials: part_rows rows of (m, l) and of hd values */
     float *part_ml, *part_acc;
     uint64_t part_rows;
+    /* the last split call wrote its outputs without partials */
+    int part_none;
     /* the stream that last used the partials: a call on another stream
        waits for its work first (part_ev), and the partials are freed only
        once it is done */
@@ -422,11 +424,18 @@ int fill_args(const janas_attn *a, int kv, SplitArgs &args, int gate_mode, const
     return JANAS_ATTN_OK;
 }
 
+/* run_split's kernels: the split kernel (1), the merge (2), and where one does
+   for both (4), that one alone */
+constexpr int kAsFits = 7;
+
 int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
-              uint32_t n_seqs, hipStream_t stream, int kernels = 3, bool fixed = false)
+              uint32_t n_seqs, hipStream_t stream, int kernels = kAsFits, bool fixed = false)
 {
     if (!split_supported(kv, a->hd))
         return JANAS_ATTN_ENOTSUP;
+    /* the merge alone, of a call that left no partials: they are made here */
+    if (kernels == 2 && a->part_none)
+        kernels = 3;
     for (uint32_t s0 = 0; s0 < n_seqs; s0 += kMaxSeqs) {
         uint32_t m = std::min(kMaxSeqs, n_seqs - s0);
         SplitArgs args;
@@ -449,7 +458,7 @@ int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
         args.once = 1;
         /* one chunk a sequence: no merge, unless it has Q8_K blocks to make or
            chunks to count */
-        bool direct = kernels == 3 && split_direct(a->hd) && !q8k && g_skip <= 0;
+        bool direct = (kernels & 4) && split_direct(a->hd) && !q8k && g_skip <= 0;
         uint32_t wg = 0, mg = 0;
         /* merge workgroups a (token, head), or a token's blocks */
         const uint32_t nd = (a->hd + args.merge_cols - 1) / args.merge_cols;
@@ -488,6 +497,8 @@ int run_split(janas_attn *a, int kv, int gate_mode, const janas_attn_seq *seqs,
             prof_end(ev, stream);
             if (e != hipSuccess)
                 return hip_err(e, "split launch");
+            if (!fixed)
+                a->part_none = direct;
         }
         if ((kernels & 2) && !direct) {
             ProfEv *ev = fixed ? nullptr : prof_begin(a, 1, stream);
@@ -1739,7 +1750,7 @@ int run_dev(janas_attn *a, int kv_type, int gate_mode, const janas_attn_seq *seq
                     shortq[ns++] = q;
             }
             if (ns) {
-                rc = run_split(a, kv_type, gate_mode, shortq, ns, st, 3, fixed);
+                rc = run_split(a, kv_type, gate_mode, shortq, ns, st, kAsFits, fixed);
                 if (rc)
                     return note(a, rc);
             }
@@ -1750,7 +1761,7 @@ int run_dev(janas_attn *a, int kv_type, int gate_mode, const janas_attn_seq *seq
             }
         }
     } else {
-        rc = run_split(a, kv_type, gate_mode, seqs, n_seqs, st, 3, fixed);
+        rc = run_split(a, kv_type, gate_mode, seqs, n_seqs, st, kAsFits, fixed);
     }
     return note(a, rc);
 }

@@ -172,3 +172,17 @@ def test_an_instance_holds_a_blocks_partials(host, geom, n_ctx):
     rows, allocs = (int(x) for x in host([f"new {h} {n_kv} {hd} 0 {n_ctx}"])[0])
     assert rows * (hd + 2) * 4 == janas_amd.part_bytes(h, n_kv, hd, max(n_ctx, 1))
     assert allocs == 2
+
+
+def test_the_merge_alone_finds_partials(host):
+    """janas_attn_run_dev_kernels: 1 and 3 leave partials, 2 merges them; after a
+    call of one chunk, whose split kernel wrote the outputs, 2 makes them first."""
+    calls = ["dev", "kernels2", "kernels2", "kernels3", "kernels2", "split", "kernels1", "kernels2",
+             "dev", "noalloc", "kernels2"]
+    want = ["split", "split merge", "merge", "split merge", "merge", "split", "split", "merge",
+            "split", "split", "split merge"]
+    got = host(["new 32 8 128 0 256"] + [f"call {c} {F16} 0 0 1 99" for c in calls])[1:]
+    assert [" ".join(x[0] for x in Call(w).launches) for w in got] == want
+    # of two chunks every call leaves them
+    got = host(["new 32 8 128 0 512", f"call dev {F16} 0 0 1 299", f"call kernels2 {F16} 0 0 1 299"])
+    assert [" ".join(x[0] for x in Call(w).launches) for w in got[1:]] == ["split merge", "merge"]
