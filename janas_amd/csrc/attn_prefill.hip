@@ -1947,10 +1947,10 @@ double prefill_tile_us(int kv, uint32_t hd, bool halves)
     if (hd > 256)
         return f16 ? 2.2 : 2.9;
     if (hd > 128)
-        return f16 ? 2.2 : kv == kI8 ? 3.4 : 2.8;
+        return f16 ? 2.2 : kv == kI8 ? 3.4 : 3.0;
     if (hd > 64)
-        return halves ? 0.92 : f16 ? 2.8 : kv == kI8 ? 3.0 : 2.75;
-    return f16 ? 1.85 : kv == kI8 ? 2.0 : 2.5;
+        return halves ? 0.92 : f16 ? 2.8 : kv == kI8 ? 3.0 : 3.1;
+    return f16 ? 1.85 : kv == kI8 ? 2.0 : 3.0;
 }
 
 hipError_t launch_prefill(int kv, const PrefillArgs &a, hipStream_t s)
