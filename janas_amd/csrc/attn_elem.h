@@ -46,39 +46,6 @@ __device__ __forceinline__ h4 lds_read_tr(const _Float16 *p)
     return __builtin_bit_cast(h4, v);
 }
 
-/* x = hi + lo, both f16; x already scaled into f16's normal range. x is
-   pinned as the f32 number it is: left free, the compiler may form hi from
-   the product that made x, rounded once to f16 (v_fma_mixlo_f16), in one
-   kernel instance and from x in another - different bits for one row in
-   two instances, and hi + lo no longer x. */
-__device__ __forceinline__ void split_hl(float x, _Float16 &hi, _Float16 &lo)
-{
-    asm volatile("" : "+v"(x));
-    hi = (_Float16)x;
-    lo = (_Float16)(x - (float)hi);
-}
-
-/* split_hl of a pair, as packed halves: the highs by one conversion, each low
-   as one multiply-add of the high half as it is, rounded once (x - hi is exact
-   in f32) - the same planes in 1.5 operations a number for the compiler's 4.
-   neg1: -1, kept out of the compiler's sight (minus_one), which would make a
-   subtraction of the multiply-add */
-__device__ __forceinline__ float minus_one()
-{
-    float m = -1.0f;
-    asm volatile("" : "+s"(m));
-    return m;
-}
-__device__ __forceinline__ void split_hl2(float x0, float x1, float neg1, h2 &hi, h2 &lo)
-{
-    asm volatile("" : "+v"(x0), "+v"(x1));
-    uint32_t w = __builtin_bit_cast(uint32_t, h2{(_Float16)x0, (_Float16)x1});
-    asm volatile("" : "+v"(w));
-    hi = __builtin_bit_cast(h2, w);
-    lo = h2{(_Float16)__builtin_fmaf((float)hi[0], neg1, x0),
-            (_Float16)__builtin_fmaf((float)hi[1], neg1, x1)};
-}
-
 /* ---- element types of the cache -------------------------------------- */
 
 /*

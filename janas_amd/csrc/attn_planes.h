@@ -1,8 +1,8 @@
 /*
- * attn_planes.h - integers of the engine's int8 / int16 caches as exact f16
- * planes, by byte permutes and packed f16 arithmetic: shared by the split
- * and wide kernels (staging a chunk) and, for int8, the exact prefill's copy
- * pass.
+ * attn_planes.h - numbers as f16 planes: the engine's int8 / int16 integers
+ * exactly, by byte permutes and packed f16 arithmetic (the split and wide
+ * kernels' staging of a chunk and, for int8, the exact prefill's copy pass),
+ * and f32 numbers as a high and a low one (f32 caches, queries, weights).
  * Internal, device code only.
  *
  * A byte b under the exponent byte 0x64 is the half 1024 + b: halves in
@@ -75,6 +75,40 @@ __device__ __forceinline__ void i16_planes8(uint32_t w0, uint32_t w1, uint32_t w
     i16_planes4(w2, w3, h1, l1);
     hi = h8{h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
     lo = h8{l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
+}
+
+/* x = hi + lo, both f16 (22 significant bits); x already scaled into f16's
+   normal range. x is pinned as the f32 number it is: left free, the compiler
+   may form hi from the product that made x, rounded once to f16
+   (v_fma_mixlo_f16), in one kernel instance and from x in another, or for lo
+   alone - different bits for one row in two instances, and hi + lo no longer x
+   (an error of 2^-10 on one weight in a hundred rows). */
+__device__ __forceinline__ void split_hl(float x, _Float16 &hi, _Float16 &lo)
+{
+    asm volatile("" : "+v"(x));
+    hi = (_Float16)x;
+    lo = (_Float16)(x - (float)hi);
+}
+
+/* split_hl of a pair, as packed halves: the highs by one conversion, each low
+   as one multiply-add of the high half as it is, rounded once (x - hi is exact
+   in f32) - the same planes in 1.5 operations a number for the compiler's 4.
+   neg1: -1, kept out of the compiler's sight (minus_one), which would make a
+   subtraction of the multiply-add */
+__device__ __forceinline__ float minus_one()
+{
+    float m = -1.0f;
+    asm volatile("" : "+s"(m));
+    return m;
+}
+__device__ __forceinline__ void split_hl2(float x0, float x1, float neg1, h2 &hi, h2 &lo)
+{
+    asm volatile("" : "+v"(x0), "+v"(x1));
+    uint32_t w = __builtin_bit_cast(uint32_t, h2{(_Float16)x0, (_Float16)x1});
+    asm volatile("" : "+v"(w));
+    hi = __builtin_bit_cast(h2, w);
+    lo = h2{(_Float16)__builtin_fmaf((float)hi[0], neg1, x0),
+            (_Float16)__builtin_fmaf((float)hi[1], neg1, x1)};
 }
 
 }  // namespace

@@ -1052,20 +1052,6 @@ __global__ __launch_bounds__(PCfg<D>::W * 64) void prefill_dma_kernel(const Pref
  * the cache itself (a 4-byte load into LDS a lane, every position clamped to
  * the rows the block sees, so nothing outside them is read).
  */
-/* x = hi + lo in f16 (22 significant bits). x is pinned in a register
-   first (an empty asm): left free, the compiler made hi from the f32
-   product x = w * vs for the products, but made it again for lo straight
-   from the exact product (v_fma_mixlo_f16 w, vs, 0: one rounding instead of
-   two) - at a rounding tie the two differ by an f16 unit, and hi + lo
-   missed the weight by twice lo (an error of 2^-10 on one weight in a
-   hundred rows). */
-__device__ __forceinline__ void split_hl(float x, _Float16 &hi, _Float16 &lo)
-{
-    asm volatile("" : "+v"(x));
-    hi = (_Float16)x;
-    lo = (_Float16)(x - (float)hi);
-}
-
 template <int EX> struct XBias {
     static constexpr float value = EX == 2 ? 14.0f : 6.0f;
 };
@@ -1260,14 +1246,11 @@ __device__ __forceinline__ void tile_pass_x(uint32_t p0, const PBlock &P, const 
 
     /* weights of value k-step ks (positions 32 (ks / 2) + 16 (ks % 2) +
        8 (e / 4) + 4 (l / 32) + e % 4), times their value scales, as two
-       planes; the sum of the weights in f32. The planes are split_hl's: a pair
-       of highs by one conversion, each low as one multiply-add of the high half
-       as it is, rounded once to f16 (x - hi is exact in f32) - the compiler's
-       own way converted each high twice and back, 5 operations a weight for
-       these 2.25; -1 is kept out of its sight or it makes a subtraction of the
-       multiply-add. int8 at 32 / 8 / 128, 8192 tokens: 941 -> 911 us */
-    float ls = 0.0f, neg1 = -1.0f;
-    asm volatile("" : "+s"(neg1));
+       planes; the sum of the weights in f32. split_hl2: the compiler's own way
+       converted each high twice and back, 5 operations a weight for its 2.25.
+       int8 at 32 / 8 / 128, 8192 tokens: 941 -> 911 us */
+    float ls = 0.0f;
+    const float neg1 = minus_one();
     auto weights = [&](int ks, h8 &ph, h8 &pl) {
 #pragma unroll
         for (int jj = 0; jj < 2; jj++) {
@@ -1294,14 +1277,12 @@ __device__ __forceinline__ void tile_pass_x(uint32_t p0, const PBlock &P, const 
                     }
                     continue;
                 }
-                asm volatile("" : "+v"(x[0]), "+v"(x[1]));
-                uint32_t hw = __builtin_bit_cast(uint32_t, h2{(_Float16)x[0], (_Float16)x[1]});
-                asm volatile("" : "+v"(hw));
-                const h2 hi = __builtin_bit_cast(h2, hw);
+                h2 hi, lo;
+                split_hl2(x[0], x[1], neg1, hi, lo);
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
                     ph[4 * jj + e + i] = hi[i];
-                    pl[4 * jj + e + i] = (_Float16)__builtin_fmaf((float)hi[i], neg1, x[i]);
+                    pl[4 * jj + e + i] = lo[i];
                 }
             }
         }
